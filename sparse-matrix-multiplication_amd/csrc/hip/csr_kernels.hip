@@ -40,10 +40,18 @@ constexpr int kWave = 64;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// T: VEC floats in registers.  Mem: the same at any float address; rows of an N
+// that is no multiple of VEC start there, and a 16-byte access needs no more.
 template <int VEC> struct Vec;
-template <> struct Vec<1> { using T = float; };
-template <> struct Vec<2> { using T = f32x2; };
-template <> struct Vec<4> { using T = f32x4; };
+template <> struct Vec<1> { using T = float; using Mem = float; };
+template <> struct Vec<2> {
+    using T = f32x2;
+    typedef f32x2 Mem __attribute__((aligned(4)));
+};
+template <> struct Vec<4> {
+    using T = f32x4;
+    typedef f32x4 Mem __attribute__((aligned(4)));
+};
 
 template <int VEC>
 __device__ __forceinline__ typename Vec<VEC>::T vzero() {
@@ -206,13 +214,22 @@ __device__ __forceinline__ typename Vec<VEC>::T load_b(__amdgpu_buffer_rsrc_t rs
         else if constexpr (VEC == 2) return sbuf_load_x2(rsrc, k, colb, 0, 0);
         else return sbuf_load_x1(rsrc, k, colb, 0, 0);
     } else {
-        return *reinterpret_cast<const typename Vec<VEC>::T*>(bcol + static_cast<size_t>(k) * N);
+        return *reinterpret_cast<const typename Vec<VEC>::Mem*>(bcol + static_cast<size_t>(k) * N);
     }
 }
 
 template <int VEC>
 __device__ __forceinline__ void store_vec(float* p, typename Vec<VEC>::T v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<typename Vec<VEC>::T*>(p));
+    __builtin_nontemporal_store(v, reinterpret_cast<typename Vec<VEC>::Mem*>(p));
+}
+
+// First column of the VEC a lane owns: col, or the row's (slice's) last VEC
+// columns when fewer than VEC are left from col on.  Those overlap the lane
+// before, which sums the same entries in the same order, so both store the same
+// bits.  Lanes past the end get that chunk too and store nothing.
+template <int VEC>
+__device__ __forceinline__ int lane_col(int col, int cend) {
+    return VEC == 1 ? min(col, cend - 1) : min(col, max(cend - VEC, 0));
 }
 
 __device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m); }
@@ -360,7 +377,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                 empty &= empty - 1;
                 float* crow = a.C + static_cast<size_t>(w0 + base + b) * N;
                 for (int c = cbeg + lane * VEC; c < cend; c += kWave * VEC) {
-                    store_vec<VEC>(crow + c, vzero<VEC>());
+                    store_vec<VEC>(crow + lane_col<VEC>(c, cend), vzero<VEC>());
                 }
             }
         }
@@ -392,11 +409,9 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
         if (one_window && pa < pb) stage(pa, pb);
 
         for (int c0 = cbeg; c0 < cend; c0 += COLS) {
-            const int  col    = c0 + glane * VEC;
-            const bool col_ok = col < cend;
-            const int  col_ld = col_ok ? col : 0;  // loads stay in bounds; never stored
-            const bool writer = grp == 0 && col_ok;
-            const float* bcol = a.B + col_ld;
+            const int  col    = lane_col<VEC>(c0 + glane * VEC, cend);
+            const bool writer = grp == 0 && c0 + glane * VEC < cend;
+            const float* bcol = a.B + col;
             if (lane == 0) s_first[wave] = (pa < pb) ? -1 : -2;
 
             int owner_row = -1;  // local row this wave finishes after the barrier
@@ -430,7 +445,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                         for (int u = 0; u < U; ++u) {
                             const int2 kv = s_kv[wave][q - win + u * G + grp];
                             vv[u] = __builtin_bit_cast(float, kv.y);
-                            bv[u] = load_b<VEC, SBUF>(rsrc, bcol, kv.x, col_ld * 4, N);
+                            bv[u] = load_b<VEC, SBUF>(rsrc, bcol, kv.x, col * 4, N);
                         }
                     };
                     // Accumulates the step starting at entry q.
@@ -768,14 +783,14 @@ __global__ __launch_bounds__(256) void csr_row_groups(RowGroupArgs a) {
         const_cast<float*>(a.B), static_cast<short>(a.N * 4), a.K, kBufWord3);
 
     for (int n0 = cbeg; n0 < cend; n0 += LC * VEC) {
-        const int  n    = n0 + c * VEC;
-        const bool col  = n < cend;  // lanes past the slice read column 0 and store nothing
+        const int  n    = lane_col<VEC>(n0 + c * VEC, cend);
+        const bool col  = n0 + c * VEC < cend;
         VT acc;
         if constexpr (COOP) {
-            acc = row_chunks_sum<VEC, U>(a, rb, start, g_end, lane & ~(L - 1), gl, e, L, LE,
-                                         col ? n * 4 : 0, L);
+            acc = row_chunks_sum<VEC, U>(a, rb, start, g_end, lane & ~(L - 1), gl, e, L, LE, n * 4,
+                                         L);
         } else {
-            acc = row_segment_sum<VEC, U>(a, rb, start + e, g_end, LE, col ? n * 4 : 0);
+            acc = row_segment_sum<VEC, U>(a, rb, start + e, g_end, LE, n * 4);
         }
         for (int m = LC; m < L; m <<= 1) acc = xor_add<VEC>(acc, m);
         if (live && !is_long && e == 0 && col) {
@@ -806,16 +821,15 @@ __global__ __launch_bounds__(256) void csr_row_groups(RowGroupArgs a) {
             const int rs = a.row_ptr[r];
             const int re = a.row_ptr[r + 1];
             for (int n0 = cbeg; n0 < cend; n0 += LC * VEC) {
-                const int  n   = n0 + c * VEC;
-                const bool col = n < cend;
+                const int  n   = lane_col<VEC>(n0 + c * VEC, cend);
+                const bool col = n0 + c * VEC < cend;
                 VT acc;
                 // One row at a time: four entries per lane in flight.
                 if constexpr (COOP) {
                     acc = row_chunks_sum<VEC, 4>(a, rb, rs + wave * kWave, re, 0, lane, we, kWave,
-                                                 WE, col ? n * 4 : 0, 4 * kWave);
+                                                 WE, n * 4, 4 * kWave);
                 } else {
-                    acc = row_segment_sum<VEC, 4>(a, rb, rs + wave * WE + we, re, 4 * WE,
-                                                  col ? n * 4 : 0);
+                    acc = row_segment_sum<VEC, 4>(a, rb, rs + wave * WE + we, re, 4 * WE, n * 4);
                 }
                 for (int m = LC; m < kWave; m <<= 1) acc = xor_add<VEC>(acc, m);
                 if (we == 0) s_part[wave][c] = acc;
@@ -847,16 +861,16 @@ bool aligned(const void* p, size_t bytes) {
     return (reinterpret_cast<uintptr_t>(p) % bytes) == 0;
 }
 
-// Widest VEC (<= want, 4 when want == 0) that keeps every lane's VEC floats
-// inside one row and naturally aligned.
-int pick_vec(int N, const float* B, float* C, int want) {
+// Widest VEC (<= want, 4 when want == 0) that a row holds once.  Rows need no
+// alignment beyond their floats (see Vec) and N need not be a multiple of VEC
+// (see lane_col): one float per lane, which other widths took before, is bound
+// by the 4x as many load instructions and lanes (MI355X, 20011 x 17001, 40 per
+// row, N = 77: 119.2 -> 32.4 us, 0.25 TB/s -> 7.6 TB/s of gathered rows).
+int pick_vec(int N, int want) {
     if (want == 0) want = 4;
-    for (int v = want; v > 1; v >>= 1) {
-        if (N % v == 0 && aligned(B, sizeof(float) * v) && aligned(C, sizeof(float) * v)) return v;
-    }
-    return 1;
+    while (want > 1 && N < want) want >>= 1;
+    return want;
 }
-
 
 // Groups per wave: enough lanes per group to cover N in one pass, at most 8
 // groups (8 lanes of 16 bytes) and at least 1 (64 lanes, several passes for
@@ -1148,7 +1162,7 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     if (want_vec != 0 && want_vec != 1 && want_vec != 2 && want_vec != 4) {
         return fail(kInvalid, "engine vec must be 1, 2 or 4");
     }
-    const int vec = pick_vec(N, B, C, want_vec);
+    const int vec = pick_vec(N, want_vec);
     // Default launches of the production roles at N of a few columns (at most
     // four column lanes of VEC floats, e.g. N <= 16 with 16-byte lanes) take
     // the sub-wave row groups: the engine keeps half or more of its lanes idle
@@ -1297,7 +1311,7 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     // then the engine, which shares long rows between eight waves with more
     // entries per step, is the safer choice.
     if (N <= 0 || M <= 0 || !b_fits_buffer(K, N)) return false;
-    const int vec    = N % 4 == 0 ? 4 : (N % 2 == 0 ? 2 : 1);
+    const int vec    = pick_vec(N, 0);
     const int slices = row_group_slices(K, N, avg_row);
     const int lc     = 1 << row_group_lc_log(M, ceil_div(ceil_div(N, slices), vec) * vec, vec);
     if (max_row > std::max(16384.0 / lc, 8.0 * avg_row)) return false;

@@ -528,3 +528,44 @@ def test_size_independent_properties_c2(S, torch, config_refs):
     assert torch.equal(c3, c1 * 2.0)
     neg = S.spmm_csr("tiled_v3", dA, -dB)
     assert torch.equal(neg, -c1)
+
+
+@pytest.mark.parametrize("N", [2, 3, 5, 6, 7, 9, 31, 33, 63, 65, 77, 127, 129, 258, 261])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_any_width_and_alignment(S, O, torch, N, shift):
+    # 16-byte lanes on rows that start at any float: the last chunk of a row
+    # overlaps the one before.  B and C start `shift` floats past an aligned
+    # address inside larger buffers whose other floats are NaN: a read outside
+    # B shows in C, a write outside C changes a NaN.
+    rng = np.random.default_rng(90 + N)
+    A = S.generate_power_law_csr(700, 900, 12.0, 1.5, 800, 91)
+    B = rng.uniform(-1, 1, (A.num_cols, N)).astype(np.float32)
+    C64, absC = O.csr_spmm_f64(A.row_ptr, A.col_idx, A.values, B)
+    dA = S.DeviceCSR(A)
+    nan = float("nan")
+    bbuf = torch.full((A.num_cols * N + 16,), nan, device="cuda")
+    dB = bbuf[4 + shift:4 + shift + A.num_cols * N].view(A.num_cols, N)
+    dB.copy_(torch.from_numpy(B))
+    parts = 7
+    rows = torch.from_numpy(S.nnz_split_rows(A, parts)).cuda()
+    bounds = torch.from_numpy(S.nnz_balanced_bounds(A, parts)).cuda()
+    E = S.EngineOptsT
+    runs = {"tiled": lambda C: S.spmm_csr("tiled", dA, dB, C),
+            "tiled_v3": lambda C: S.spmm_csr("tiled_v3", dA, dB, C),
+            "engine": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(0, 4), C),
+            "slices": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(0, 0, 0, 0, 0, 4), C),
+            "pointers": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(0, 0, 0, 0, 0, 0, 1), C),
+            "hint": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(max_row_hint=12), C),
+            "groups": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(row_groups=2), C),
+            "coop": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(row_groups=3, slices=2), C),
+            "split": lambda C: S.spmm_tiled_v3_split(dA, rows, dB, C),
+            "noalloc": lambda C: S.spmm_tiled_v3_split_noalloc(dA, rows, dB, C),
+            "bounds": lambda C: S.spmm_tiled_v3_partitioned(dA, bounds, dB, C)}
+    for name, run in runs.items():
+        say(f"csr any width {name} N={N} shift={shift}")
+        cbuf = torch.full((A.num_rows * N + 16,), nan, device="cuda")
+        dC = cbuf[4 + shift:4 + shift + A.num_rows * N].view(A.num_rows, N)
+        run(dC)
+        torch.cuda.synchronize()
+        check_csr(dC.cpu().numpy(), C64, absC)
+        assert torch.isnan(cbuf[:4 + shift]).all() and torch.isnan(cbuf[4 + shift + dC.numel():]).all()
