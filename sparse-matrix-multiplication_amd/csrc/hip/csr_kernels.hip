@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "engine.h"
 #include "spmm/utils.h"
@@ -119,85 +120,107 @@ __global__ __launch_bounds__(256, MIN_WAVES_PER_EU) void csr_wave_per_row(
 //
 // Partition.  Workgroup g owns rows [r_begin, r_end): either g*R .. g*R+R
 // (implicit, R chosen from the average row length) or bounds[g] .. bounds[g+1]
-// (an explicit nnz-balanced partition).  Inside the workgroup the nonzeros of
-// those rows are cut into WAVES equal contiguous ranges, one per wave, so a
-// long row is shared by several waves and many short rows by one wave.
-// Merge-path mode (split_rows) cuts at the workgroup level too: workgroup g
-// takes nonzeros [nnz*g/P, nnz*(g+1)/P) whatever rows they belong to; a row
-// that began in an earlier workgroup is summed into carry[g] instead of C, and
-// csr_split_fixup adds the carries to C in part order afterwards.
+// (an explicit nnz-balanced partition).  Merge-path mode (split_rows) cuts at
+// the workgroup level too: workgroup g takes nonzeros [nnz*g/P, nnz*(g+1)/P)
+// whatever rows they belong to; a row that began in an earlier workgroup is
+// summed into carry[g] instead of C, and csr_split_fixup adds the carries to C
+// in part order afterwards.
 //
-// Lane groups.  A wave is split into G groups of 64/G lanes; each group covers
-// one column tile of COLS = (64/G) * VEC columns with VEC-float (up to 16-byte)
-// loads, and the groups take interleaved entries of the wave's range (group h
-// takes entries h, h+G, h+2G, ...).  One load instruction therefore fetches G
-// different B row segments: for N = 128 fp32, G = 2 and each half-wave reads
-// one 512-byte row with dwordx4 loads.
+// Lane groups.  A wave is split into G groups of L lanes, any L that covers the
+// columns of a pass with VEC-float (up to 16-byte) loads: 20 lanes and three
+// groups for N = 77, eight lanes and eight groups for a slice of 32 columns.
+// The nonzeros of the workgroup are cut into equal contiguous ranges, one per
+// group, so a long row is shared by several groups and a group may take many
+// short rows.  One load instruction fetches G different B row segments, and no
+// group waits for another's row end: at one of its own a group stores (or puts
+// aside) its sum under its lanes' mask and goes on.
 //
-// Per wave.  The wave copies (col, value) pairs of its range into its own LDS
-// window (kWCap entries, all loads issued at once); every lane then reads the
-// entry of its group with one broadcast ds_read_b64 and gathers its B segment
-// with a bounds-checked buffer load (one record per B row, so the row index is
-// the load's index operand and needs no address arithmetic).  The range is
-// walked in steps of U*G entries with the next step's loads in flight while
-// the current step is accumulated.  A scalar test per step sends only the
-// steps that cross a row end to the slow path, so row bookkeeping costs per
-// row, not per entry (measured on MI355X: per-entry scalar tests made the
-// kernel issue-bound on the shared scalar unit).  At a row end the groups'
-// tiles are summed with cross-lane shuffles and the row is flushed:
-//   - a row that lies wholly inside the wave's range is stored to C;
-//   - the first row of a range that started in an earlier wave goes to an LDS
-//     slot (s_part[wave]);
-//   - the last row of a range that continues in a later wave stays in the
+// Per wave.  The wave copies (col, value) pairs of its groups' ranges into its
+// LDS window (kWCap entries, one run per group, all loads issued at once);
+// every lane then reads the entry of its group with a broadcast ds_read_b64 and
+// gathers its B segment with a bounds-checked buffer load (one record per B
+// row, so the row index is the load's index operand and needs no address
+// arithmetic).  Each register of the U rows in flight is refilled as soon as it
+// is used, and the entries are read from LDS one step ahead.  At a row's end:
+//   - a row that lies wholly inside the group's range is stored to C;
+//   - the first row of a range that started in an earlier group goes to an LDS
+//     slot of the group;
+//   - the last row of a range that continues in a later group stays in the
 //     registers of its owner, which after a barrier adds the LDS slots of the
-//     following waves in wave order and stores it.
+//     following groups in order and stores it.
 // The sum order is fixed by the partition and the launch shape, so results
 // are deterministic run to run.
+//
+// What bounds it: the lines a CU has in flight towards L2 (20 TB/s of gathered
+// rows at best where B fits the L2s), and past the L2s their misses (8 - 10
+// TB/s).  Measured on MI355X against the form before it, in which the groups of
+// a wave took alternate entries of one range, in whole steps of U * G entries,
+// and reduced at every row end (csr_rowblock_wide is that form): 20011 x 17001,
+// 40 per row, N = 77 30.8 -> 23.7 us; 65536^2, 32 per row, N = 256 250 -> 211 us
+// with eight slices (298 in the old form, whose steps of 32 entries each held a
+// row end); power-law 65536^2, N = 32 over B-row halves 67 -> 35 us; 8192^2
+// power-law, N = 256 49.6 -> 29.1 us; 1.25x over 300 uniform and power-law
+// inputs.
 //
 // Rows of the workgroup without nonzeros are zero-filled up front.  Row
 // pointers are staged in LDS in windows of kRpCap rows.
 // ---------------------------------------------------------------------------
-struct RowblockArgs {
+// One sparse matrix, its B, its C and (merge-path) its partition.
+struct RowblockPart {
     const int*   row_ptr;
     const int*   col_idx;
     const float* vals;
     const float* B;
     float*       C;
-    const int*   bounds;  // nullable
-    int          M;
-    int          N;
-    int          K;            // rows of B (records of the B buffer)
-    int          rows_per_block;
-    int          nblocks;      // row blocks (workgroups of one column slice)
-    int          slices;       // column slices: 1, 2, 4 or 8
-    int          slice_cols;   // columns per slice (a multiple of VEC)
     // Merge-path partition (nullable split_rows): part g = nonzeros
     // [nnz*g/nblocks, nnz*(g+1)/nblocks); split_rows[g] is the row holding the
     // first of them (split_rows[0] = 0, split_rows[nblocks] = M); carry is a
     // nblocks x N workspace for the partial of a part's first row when that
     // row began in an earlier part.
-    const int*   split_rows;
-    float*       carry;
-    long long    nnz;
-    // B-row halves (merge-path only): workgroups on XCDs 4-7 take this second
-    // descriptor -- the entries of A whose columns lie in B's upper rows, with
+    const int*   split_rows = nullptr;
+    float*       carry = nullptr;
+    long long    nnz = 0;
+    int          K = 0;        // rows of B (records of the B buffer)
+    int          nblocks = 0;  // row blocks (workgroups of one column slice)
+};
+
+struct RowblockArgs {
+    RowblockPart part;
+    const int*   bounds = nullptr;    // nullable: rows of each row block
+    int          M = 0;
+    int          N = 0;
+    int          rows_per_block = 0;
+    int          slices = 1;          // column slices: 1, 2, 4 or 8
+    int          slice_cols = 0;      // columns per slice (a multiple of VEC)
+    int          group_lanes = 64;    // lanes per group
+    int          groups = 1;          // groups per wave: at most 64 / group_lanes
+    int          window_log = 0;      // log2 of the entries a group stages at a time
+    int          lanes_inv = 0;       // lane / group_lanes == lane * lanes_inv >> 16
+    unsigned     groups_inv = 0;      // 2^32 / groups, rounded up
+    // B-row halves only (merge-path only): workgroups on XCDs 4-7 take this
+    // part -- the entries of A whose columns lie in B's upper rows, with
     // rebased columns, those B rows, their own output and merge-path table --
     // and XCDs 0-3 the first, so each XCD's L2 holds half of B at full width.
-    int          halves = 0;
-    const int*   row_ptr1 = nullptr;
-    const int*   col_idx1 = nullptr;
-    const float* vals1 = nullptr;
-    const float* B1 = nullptr;
-    float*       C1 = nullptr;
-    int          K1 = 0;
-    const int*   split_rows1 = nullptr;
-    float*       carry1 = nullptr;
-    long long    nnz1 = 0;
-    int          nblocks1 = 0;
+    // Last, so that the other launches read two cache lines less.
+    RowblockPart upper{};
 };
+
+// Has every argument loaded before the first branch on one of them.  Left to
+// itself the compiler loads each group of arguments where it is first needed,
+// and every group costs a small launch one more wait on the scalar cache
+// (MI355X, 2048^2, 40 per row, N = 256: 6.84 against 6.63 us).
+__device__ __forceinline__ void load_args(const RowblockArgs& a, const RowblockPart& m) {
+    asm volatile("" ::"s"(m.row_ptr), "s"(m.col_idx), "s"(m.vals), "s"(m.B), "s"(m.C),
+                 "s"(m.split_rows), "s"(m.carry), "s"(m.nnz), "s"(m.K), "s"(m.nblocks),
+                 "s"(a.bounds), "s"(a.M), "s"(a.N), "s"(a.rows_per_block), "s"(a.slices),
+                 "s"(a.slice_cols), "s"(a.group_lanes), "s"(a.groups), "s"(a.window_log),
+                 "s"(a.lanes_inv), "s"(a.groups_inv));
+}
 
 constexpr int kRpCap = 1024;  // row pointers staged per window
 constexpr int kWCap  = 256;   // (col, value) entries a wave stages at a time
+constexpr int kMinWindow = 16;  // entries of a group's window: two steps
+constexpr int kMaxGroups = kWCap / kMinWindow;  // lane groups of a wave
 
 // Third dword of a gfx9 buffer resource: 32-bit data format, no swizzle.
 constexpr int kBufWord3 = 0x00020000;
@@ -234,28 +257,6 @@ __device__ __forceinline__ int lane_col(int col, int cend) {
 
 __device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m); }
 
-// Sum of the G groups' tiles, returned to every lane.
-template <int VEC, int G>
-__device__ __forceinline__ typename Vec<VEC>::T reduce_groups(typename Vec<VEC>::T v) {
-    if constexpr (G == 1) {
-        return v;
-    } else {
-        using VT = typename Vec<VEC>::T;
-#pragma unroll
-        for (int m = kWave / G; m < kWave; m <<= 1) {
-            VT o;
-            if constexpr (VEC == 1) {
-                o = shfl_xor_f(v, m);
-            } else {
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] = shfl_xor_f(v[e], m);
-            }
-            v += o;
-        }
-        return v;
-    }
-}
-
 // Orders a wave's LDS writes before its own lanes' reads of them.
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -263,24 +264,42 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int VEC, int G, int WAVES, int U, bool SBUF>
+// One staged entry of A: the B row in the low half, the value in the high one
+// (a single 8-byte LDS read; as two fields the compiler reads them apart).
+typedef uint64_t Entry;
+__device__ __forceinline__ Entry entry(int k, float v) {
+    return static_cast<uint32_t>(k) | (static_cast<Entry>(__builtin_bit_cast(uint32_t, v)) << 32);
+}
+__device__ __forceinline__ int entry_row(Entry e) { return static_cast<int>(e); }
+__device__ __forceinline__ float entry_value(Entry e) {
+    return __builtin_bit_cast(float, static_cast<uint32_t>(e >> 32));
+}
+
+template <int VEC, int WAVES, int U, bool SBUF, bool HALVES>
 __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     using VT = typename Vec<VEC>::T;
-    constexpr int LPG  = kWave / G;   // lanes per group
-    constexpr int COLS = LPG * VEC;   // columns per pass
-    constexpr int STEP = U * G;       // entries per step
-    static_assert(kWave % STEP == 0 && kWCap % kWave == 0, "U * G must divide the wave size");
+    static_assert(kWCap % kWave == 0 && kMinWindow % U == 0, "whole steps per window");
 
-    __shared__ int  s_rp[kRpCap + 1];
-    __shared__ VT   s_part[WAVES][LPG];
-    __shared__ int  s_first[WAVES];
-    __shared__ int2 s_kv[WAVES][kWCap + STEP];
+    __shared__ int  s_rp[kRpCap + 2];
+    __shared__ VT   s_part[WAVES * kWave];   // by group and lane: the group's head piece
+    __shared__ int  s_first[WAVES * kWave];  // by group: see below
+    __shared__ Entry s_kv[WAVES][kWCap + kMaxGroups * (2 * U + 1)];
 
+    load_args(a, a.part);
     const int lane  = threadIdx.x & (kWave - 1);
     const int wave  = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int grp   = lane / LPG;
-    const int glane = lane % LPG;
+    const int lpg   = a.group_lanes;
+    const int G     = a.groups;
+    // Lanes past the last group shadow its last lane and never store.
+    const int grp   = min(lane * a.lanes_inv >> 16, G - 1);
+    const int glane = min(lane - grp * lpg, lpg - 1);
+    const bool live = lane < G * lpg;
+    const int gi    = wave * G + grp;  // group of the workgroup
+    const int NG    = WAVES * G;
+    VT* const my_part = s_part + gi * lpg + glane;
     const int N     = a.N;
+    const int cap   = 1 << a.window_log;  // entries a group stages at a time
+    const int cols  = lpg * VEC;          // columns per pass
 
     // Column slices are tied to XCDs: workgroups are dispatched round-robin
     // over the 8 XCDs, so workgroup g runs on XCD g % 8.  With S slices, XCDs
@@ -288,43 +307,33 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     // block, so each XCD's L2 holds only 1/S of B.  With B-row halves, XCDs
     // 0-3 work through the parts of the first descriptor and XCDs 4-7 through
     // those of the second (all columns each).
-    int rb = blockIdx.x, slice = 0;
-    if (a.halves) {
+    int rb = blockIdx.x, slice = 0, half = 0;
+    if constexpr (HALVES) {
         const int x = blockIdx.x & 7;
-        rb = (blockIdx.x >> 3) * 4 + (x & 3);
-        if (x >= 4) {
-            a.row_ptr    = a.row_ptr1;
-            a.col_idx    = a.col_idx1;
-            a.vals       = a.vals1;
-            a.B          = a.B1;
-            a.C          = a.C1;
-            a.K          = a.K1;
-            a.split_rows = a.split_rows1;
-            a.carry      = a.carry1;
-            a.nnz        = a.nnz1;
-            a.nblocks    = a.nblocks1;
-        }
+        rb   = (blockIdx.x >> 3) * 4 + (x & 3);
+        half = x >> 2;
     } else if (a.slices > 1) {
         const int per = 8 / a.slices;  // XCDs per slice
         const int x   = blockIdx.x & 7;
         rb    = (blockIdx.x >> 3) * per + x % per;
         slice = x / per;
     }
-    if (rb >= a.nblocks) return;  // whole workgroup, before any barrier
+    const RowblockPart m = HALVES && half ? a.upper : a.part;
+    if (rb >= m.nblocks) return;  // whole workgroup, before any barrier
     const int cbeg = slice * a.slice_cols;
     const int cend = min(N, cbeg + a.slice_cols);
 
     int r_begin, r_end, zero_end;
-    const bool split = a.split_rows != nullptr;
+    const bool split = m.split_rows != nullptr;
     long long nz_lo = 0, nz_hi = 0;
     int wg_head = -1;  // first row, when it began in an earlier part (merge-path only)
     if (split) {
-        nz_lo    = a.nnz * rb / a.nblocks;
-        nz_hi    = a.nnz * (rb + 1) / a.nblocks;
-        r_begin  = a.split_rows[rb];
-        zero_end = a.split_rows[rb + 1];          // empty rows [r_begin, zero_end) are ours
+        nz_lo    = m.nnz * rb / m.nblocks;
+        nz_hi    = m.nnz * (rb + 1) / m.nblocks;
+        r_begin  = m.split_rows[rb];
+        zero_end = m.split_rows[rb + 1];          // empty rows [r_begin, zero_end) are ours
         r_end    = min(a.M, zero_end + 1);         // + the row our last nonzeros start
-        if (nz_lo < nz_hi && r_begin < a.M && a.row_ptr[r_begin] < nz_lo) wg_head = r_begin;
+        if (nz_lo < nz_hi && r_begin < a.M && m.row_ptr[r_begin] < nz_lo) wg_head = r_begin;
     } else if (a.bounds != nullptr) {
         r_begin  = a.bounds[rb];
         r_end    = a.bounds[rb + 1];
@@ -336,7 +345,310 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     }
 
     __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(a.B), static_cast<short>(SBUF ? N * 4 : 0), SBUF ? a.K : 0, kBufWord3);
+        const_cast<float*>(m.B), static_cast<short>(SBUF ? N * 4 : 0), SBUF ? m.K : 0, kBufWord3);
+    Entry* const kv = s_kv[wave];
+    // A group's window and the 2U empty entries that the last steps' loads may
+    // read; an odd stride puts the groups' windows on different banks.
+    const int kv_len  = cap + 2 * U + 1;
+    const int kv_mine = grp * kv_len;
+    for (int i = glane; i <= 2 * U; i += lpg) kv[kv_mine + cap + i] = entry(SBUF ? -1 : 0, 0.0f);
+
+    for (int w0 = r_begin; w0 < r_end; w0 += kRpCap) {
+        const int nr = min(r_end - w0, kRpCap);
+        __syncthreads();  // the previous window is no longer read
+        for (int i = threadIdx.x; i <= nr; i += WAVES * kWave) s_rp[i] = m.row_ptr[w0 + i];
+        __syncthreads();
+
+        // Zero-fill the rows of this window that hold no nonzeros.
+        for (int base = wave * kWave; base < nr; base += WAVES * kWave) {
+            const int i = base + lane;
+            uint64_t empty = __ballot(i < nr && w0 + i < zero_end && s_rp[i] == s_rp[i + 1]);
+            while (empty) {
+                const int b = __builtin_ctzll(empty);
+                empty &= empty - 1;
+                float* crow = m.C + static_cast<size_t>(w0 + base + b) * N;
+                for (int c = cbeg + lane * VEC; c < cend; c += kWave * VEC) {
+                    store_vec<VEC>(crow + lane_col<VEC>(c, cend), vzero<VEC>());
+                }
+            }
+        }
+
+        int nz0 = s_rp[0];
+        int nz_end = s_rp[nr];
+        if (split) {
+            nz0    = static_cast<int>(max(static_cast<long long>(nz0), nz_lo));
+            nz_end = static_cast<int>(min(static_cast<long long>(nz_end), nz_hi));
+        }
+        const int total = nz_end - nz0;
+        if (total <= 0) continue;  // uniform across the workgroup
+        // Entries per group: an equal share, in whole steps (total / NG or
+        // just over, by the reciprocal).
+        const int share =
+            (static_cast<int>(__umulhi(total, a.groups_inv)) / WAVES + U) / U * U;
+        const unsigned rest = total;
+        const unsigned from = min(rest, static_cast<unsigned>(wave * G) * share);  // the wave's first
+        const int pa   = nz0 + static_cast<int>(min(rest, static_cast<unsigned>(gi) * share));
+        const int pb   = nz0 + static_cast<int>(min(rest, static_cast<unsigned>(gi + 1) * share));
+        const int wlen = static_cast<int>(min<unsigned>(share, rest - from));  // its longest range
+
+        // First local row: the last i in [0, nr) with s_rp[i] <= pa.
+        int first = 0;
+        {
+            int lo = 0, hi = nr - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (s_rp[mid] <= pa) lo = mid; else hi = mid - 1;
+            }
+            first = lo;
+        }
+
+        // Copies entries win .. win + cap - 1 of each group's range into the
+        // groups' LDS windows, one coalesced run per group, all loads issued
+        // before the first LDS write.  Slots past a group's range hold record
+        // -1 (reads zeros) and value 0.
+        const char* cols_at = reinterpret_cast<const char*>(m.col_idx + nz0 + from);
+        const char* vals_at = reinterpret_cast<const char*>(m.vals + nz0 + from);
+        auto stage = [&](int win) {
+            constexpr int NL = kWCap / kWave;
+            int   kk[NL];
+            float vx[NL];
+            int   l = lane;
+            asm volatile("" : "+v"(l));  // keeps the slot arithmetic out of the entry loop's registers
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                const int idx = i * kWave + l;
+                const int off = win + (idx & (cap - 1));
+                const unsigned e  = static_cast<unsigned>(idx >> a.window_log) * share + off;
+                const bool     in = off < share && e < rest - from;
+                const unsigned at = (in ? e : 0u) * 4u;
+                kk[i] = *reinterpret_cast<const int*>(cols_at + at);
+                vx[i] = *reinterpret_cast<const float*>(vals_at + at);
+                if (!in) {
+                    kk[i] = SBUF ? -1 : 0;
+                    vx[i] = 0.0f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                const int idx = i * kWave + l;
+                const int h   = idx >> a.window_log;
+                if (h < G) {
+                    kv[h * kv_len + (idx & (cap - 1))] =
+                        entry(kk[i], vx[i]);
+                }
+            }
+            wave_lds_sync();
+        };
+
+        // A range that fits one window is staged once for all column passes.
+        const bool one_window = wlen <= cap;
+        if (wlen > 0 && one_window) stage(0);
+
+        for (int c0 = cbeg; c0 < cend; c0 += cols) {
+            const int  col    = lane_col<VEC>(c0 + glane * VEC, cend);
+            const bool writer = live && c0 + glane * VEC < cend;
+            const float* bcol = m.B + col;
+            if (live && glane == 0) s_first[gi] = -1;
+
+            int owner_row = -1;  // local row this group finishes after the barrier
+            VT acc = vzero<VEC>();
+            if (wlen > 0) {
+                int  row  = first;
+                bool head = s_rp[row] < pa;  // row began in an earlier group
+                // Where the row ends inside the range (counted from its
+                // start), or never.
+                int row_len;
+                {
+                    const int e = s_rp[row + 1];
+                    row_len = e < pb ? e - pa : 0x7fffffff;
+                }
+
+                int next_end = s_rp[row + 2 <= nr ? row + 2 : nr];
+
+                auto flush = [&](int at) {
+                    if (head) {
+                        if (live) *my_part = acc;
+                        if (live && glane == 0) s_first[gi] = row;
+                        head = false;
+                    } else if (writer) {
+                        store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, acc);
+                    }
+                    acc = vzero<VEC>();
+                    ++row;
+                    int e = next_end;
+                    while (e <= at + pa && row < nr - 1) {  // empty rows
+                        ++row;
+                        e = s_rp[row + 1];
+                    }
+                    next_end = s_rp[min(row + 2, nr)];
+                    row_len = e < pb ? e - pa : 0x7fffffff;
+                };
+
+                for (int win = 0; win < wlen; win += cap) {
+                    if (!one_window) stage(win);
+                    const int n = min(cap, wlen - win);
+
+                    // U rows in flight per group, each register refilled as
+                    // soon as it is used; the entries of the next step are
+                    // read from LDS one step ahead.
+                    VT    bv[U];
+                    float vv[U];
+                    Entry next[U];
+                    int at_kv = kv_mine;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        vv[u] = entry_value(kv[at_kv + u]);
+                        bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(kv[at_kv + u]), col * 4, N);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) next[u] = kv[at_kv + U + u];
+                    // Only the row end branches, never the loads: values loaded
+                    // on two paths would have to arrive before the paths join.
+                    auto step = [&](int at0, auto refill) {
+                        const bool ends = __ballot(row_len < at0 + U) != 0;
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            if (__builtin_expect(ends, 0)) {
+                                if (at0 + u == row_len) flush(at0 + u);
+                            }
+                            if (SBUF || at0 + u < pb - pa) acc = vv[u] * bv[u] + acc;
+                            if constexpr (decltype(refill)::value) {
+                                __builtin_amdgcn_sched_barrier(0);  // into the registers just used
+                                vv[u] = entry_value(next[u]);
+                                bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(next[u]), col * 4, N);
+                                next[u] = kv[at_kv + 2 * U + u];
+                                __builtin_amdgcn_sched_barrier(0);  // a step ahead of its use
+                            }
+                        }
+                    };
+                    int q = 0;
+                    for (; q + U < n; q += U) {
+                        step(win + q, std::true_type());
+                        at_kv += U;
+                        asm volatile("" : "+v"(at_kv));  // one address, the reads at constant offsets
+                    }
+                    step(win + q, std::false_type());
+                }
+                // The row being accumulated when the range ends.
+                if (pa < pb) {
+                    if (head) {
+                        if (live) *my_part = acc;
+                        if (live && glane == 0) s_first[gi] = row;
+                    } else if (s_rp[row + 1] <= pb) {
+                        if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, acc);
+                    } else {
+                        owner_row = row;
+                    }
+                }
+            }
+            __syncthreads();
+            if (owner_row >= 0) {
+                for (int w = gi + 1; w < NG; ++w) {
+                    if (s_first[w] != owner_row) break;
+                    acc += s_part[w * lpg + glane];
+                }
+                if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + owner_row) * N + col, acc);
+            }
+            if (wg_head >= 0 && w0 == r_begin && gi == 0) {
+                // The part's first row began in an earlier part: the groups that
+                // hold pieces of it (local row 0, leading groups) go to the carry.
+                VT sum = vzero<VEC>();
+                for (int w = 0; w < NG; ++w) {
+                    if (s_first[w] != 0) break;
+                    sum += s_part[w * lpg + glane];
+                }
+                if (writer) store_vec<VEC>(m.carry + static_cast<size_t>(rb) * N + col, sum);
+            }
+            __syncthreads();  // s_part / s_first are rewritten by the next column pass
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The engine on wide B (one or two lane groups per wave) where the partition
+// is balanced beforehand: merge-path parts, and rows that the caller's longest
+// row shows to be even.  As csr_rowblock, except that the groups of a wave take
+// alternate entries of one range instead of a range each, in steps of U * G
+// entries with the next step's loads issued before the current one is used, and
+// sum their tiles with xor shuffles at a row end.  A scalar test per step sends
+// only the steps that hold a row end to the slow path, so this form spends less
+// per entry and starts half as many row pieces; csr_rowblock's groups wait for
+// nobody and win from three groups on and on uneven rows.  MI355X, this form
+// against csr_rowblock: 16384^2 power-law over B-row halves, N = 128 61.3 against
+// 62.7 us; 8192^2, 100 per row, N = 256 36.6 against 37.6; 2048^2, 250 per row,
+// N = 256 18.9 against 19.9; merge-path 8192^2 power-law, N = 32 (eight groups)
+// 19.0 against 14.2.
+// ---------------------------------------------------------------------------
+// Sum of the G groups' tiles, returned to every lane.
+template <int G>
+__device__ __forceinline__ f32x4 reduce_groups(f32x4 v) {
+#pragma unroll
+    for (int m = kWave / G; m < kWave; m <<= 1) {
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = shfl_xor_f(v[e], m);
+        v += o;
+    }
+    return v;
+}
+
+template <int G, int WAVES, bool HALVES>
+__global__ __launch_bounds__(WAVES * 64) void csr_rowblock_wide(RowblockArgs a) {
+    constexpr int VEC = 4, U = 4;
+    using VT = f32x4;
+    constexpr int LPG  = kWave / G;   // lanes per group
+    constexpr int COLS = LPG * VEC;   // columns per pass
+    constexpr int STEP = U * G;       // entries per step
+    static_assert(kWave % STEP == 0 && kWCap % kWave == 0, "U * G must divide the wave size");
+
+    __shared__ int  s_rp[kRpCap + 1];
+    __shared__ VT   s_part[WAVES][LPG];
+    __shared__ int  s_first[WAVES];
+    __shared__ int2 s_kv[WAVES][kWCap + STEP];
+
+    load_args(a, a.part);
+    const int lane  = threadIdx.x & (kWave - 1);
+    const int wave  = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp   = lane / LPG;
+    const int glane = lane % LPG;
+    const int N     = a.N;
+
+    // Column slices and B-row halves as in csr_rowblock.
+    int rb = blockIdx.x, slice = 0, half = 0;
+    if constexpr (HALVES) {
+        const int x = blockIdx.x & 7;
+        rb   = (blockIdx.x >> 3) * 4 + (x & 3);
+        half = x >> 2;
+    } else if (a.slices > 1) {
+        const int per = 8 / a.slices;
+        const int x   = blockIdx.x & 7;
+        rb    = (blockIdx.x >> 3) * per + x % per;
+        slice = x / per;
+    }
+    const RowblockPart m = HALVES && half ? a.upper : a.part;
+    if (rb >= m.nblocks) return;  // whole workgroup, before any barrier
+    const int cbeg = slice * a.slice_cols;
+    const int cend = min(N, cbeg + a.slice_cols);
+
+    int r_begin, r_end, zero_end;
+    const bool split = m.split_rows != nullptr;
+    long long nz_lo = 0, nz_hi = 0;
+    int wg_head = -1;  // first row, when it began in an earlier part (merge-path only)
+    if (split) {
+        nz_lo    = m.nnz * rb / m.nblocks;
+        nz_hi    = m.nnz * (rb + 1) / m.nblocks;
+        r_begin  = m.split_rows[rb];
+        zero_end = m.split_rows[rb + 1];          // empty rows [r_begin, zero_end) are ours
+        r_end    = min(a.M, zero_end + 1);         // + the row our last nonzeros start
+        if (nz_lo < nz_hi && r_begin < a.M && m.row_ptr[r_begin] < nz_lo) wg_head = r_begin;
+    } else {
+        r_begin  = rb * a.rows_per_block;
+        r_end    = min(a.M, r_begin + a.rows_per_block);
+        zero_end = r_end;
+    }
+
+    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(m.B), static_cast<short>(N * 4), m.K, kBufWord3);
     // Entries past a window's end read by the masked lanes of its last step.
     for (int i = lane; i < STEP; i += kWave) s_kv[wave][kWCap + i] = make_int2(0, 0);
 
@@ -350,8 +662,8 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int e = min(lo + i * kWave + lane, hi - 1);
-            kk[i] = a.col_idx[e];
-            vx[i] = a.vals[e];
+            kk[i] = m.col_idx[e];
+            vx[i] = m.vals[e];
         }
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
@@ -365,7 +677,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     for (int w0 = r_begin; w0 < r_end; w0 += kRpCap) {
         const int nr = min(r_end - w0, kRpCap);
         __syncthreads();  // the previous window is no longer read
-        for (int i = threadIdx.x; i <= nr; i += WAVES * kWave) s_rp[i] = a.row_ptr[w0 + i];
+        for (int i = threadIdx.x; i <= nr; i += WAVES * kWave) s_rp[i] = m.row_ptr[w0 + i];
         __syncthreads();
 
         // Zero-fill the rows of this window that hold no nonzeros.
@@ -375,7 +687,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
             while (empty) {
                 const int b = __builtin_ctzll(empty);
                 empty &= empty - 1;
-                float* crow = a.C + static_cast<size_t>(w0 + base + b) * N;
+                float* crow = m.C + static_cast<size_t>(w0 + base + b) * N;
                 for (int c = cbeg + lane * VEC; c < cend; c += kWave * VEC) {
                     store_vec<VEC>(crow + lane_col<VEC>(c, cend), vzero<VEC>());
                 }
@@ -411,7 +723,6 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
         for (int c0 = cbeg; c0 < cend; c0 += COLS) {
             const int  col    = lane_col<VEC>(c0 + glane * VEC, cend);
             const bool writer = grp == 0 && c0 + glane * VEC < cend;
-            const float* bcol = a.B + col;
             if (lane == 0) s_first[wave] = (pa < pb) ? -1 : -2;
 
             int owner_row = -1;  // local row this wave finishes after the barrier
@@ -422,13 +733,13 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                 bool head    = s_rp[row] < pa;  // row began in an earlier wave
 
                 auto flush = [&]() {
-                    const VT t = reduce_groups<VEC, G>(acc);
+                    const VT t = reduce_groups<G>(acc);
                     if (head) {
                         if (grp == 0) s_part[wave][glane] = t;
                         if (lane == 0) s_first[wave] = row;
                         head = false;
                     } else if (writer) {
-                        store_vec<VEC>(a.C + static_cast<size_t>(w0 + row) * N + col, t);
+                        store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, t);
                     }
                     acc = vzero<VEC>();
                 };
@@ -445,7 +756,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                         for (int u = 0; u < U; ++u) {
                             const int2 kv = s_kv[wave][q - win + u * G + grp];
                             vv[u] = __builtin_bit_cast(float, kv.y);
-                            bv[u] = load_b<VEC, SBUF>(rsrc, bcol, kv.x, col * 4, N);
+                            bv[u] = load_b<VEC, true>(rsrc, nullptr, kv.x, col * 4, N);
                         }
                     };
                     // Accumulates the step starting at entry q.
@@ -484,9 +795,9 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                     }
                 }
                 // The row being accumulated when the range ends.
-                acc = reduce_groups<VEC, G>(acc);
+                acc = reduce_groups<G>(acc);
                 if (row_end == pb && !head) {
-                    if (writer) store_vec<VEC>(a.C + static_cast<size_t>(w0 + row) * N + col, acc);
+                    if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, acc);
                 } else if (head) {
                     if (grp == 0) s_part[wave][glane] = acc;
                     if (lane == 0) s_first[wave] = row;
@@ -502,7 +813,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                     if (f != owner_row) break;
                     acc += s_part[w][glane];
                 }
-                if (writer) store_vec<VEC>(a.C + static_cast<size_t>(w0 + owner_row) * N + col, acc);
+                if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + owner_row) * N + col, acc);
             }
             if (wg_head >= 0 && w0 == r_begin && wave == 0) {
                 // The part's first row began in an earlier part: the waves that
@@ -514,7 +825,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                     if (f != 0) break;
                     sum += s_part[w][glane];
                 }
-                if (writer) store_vec<VEC>(a.carry + static_cast<size_t>(rb) * N + col, sum);
+                if (writer) store_vec<VEC>(m.carry + static_cast<size_t>(rb) * N + col, sum);
             }
             __syncthreads();  // s_part / s_first are rewritten by the next column pass
         }
@@ -872,67 +1183,96 @@ int pick_vec(int N, int want) {
     return want;
 }
 
-// Groups per wave: enough lanes per group to cover N in one pass, at most 8
-// groups (8 lanes of 16 bytes) and at least 1 (64 lanes, several passes for
-// wide N).
-int pick_groups(int N, int vec, int want) {
-    if (want == 1 || want == 2 || want == 4 || (want == 8 && vec == 4)) return want;
-    const int lanes = (N + vec - 1) / vec;
-    if (lanes <= 8 && vec == 4) return 8;
-    if (lanes <= 16) return 4;
-    if (lanes <= 32) return 2;
-    return 1;
+// Lane groups of a wave: with L = lanes of one row (slice) and p column passes
+// a group takes ceil(L / p) lanes; the pass count with the fewest passes per
+// entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
+void set_groups(RowblockArgs& a, int cols, int vec, int want) {
+    const int lanes = ceil_div(cols, vec);
+    if (want == 1 || want == 2 || want == 4 || (want == 8 && vec == 4)) {
+        a.groups      = want;
+        a.group_lanes = kWave / want;
+    } else {
+        int passes = ceil_div(lanes, kWave), best = passes;
+        const auto groups_of = [&](int p) {
+            return std::min(kMaxGroups, kWave / ceil_div(lanes, p));
+        };
+        for (int p = passes + 1; p <= 2 * passes; ++p) {
+            if (4 * p * groups_of(best) < 3 * best * groups_of(p)) best = p;
+        }
+        a.group_lanes = ceil_div(lanes, best);
+        a.groups      = groups_of(best);
+    }
+    a.lanes_inv  = ceil_div(1 << 16, a.group_lanes);
+    a.groups_inv = static_cast<unsigned>(
+        std::min<unsigned long long>(0xffffffffull, ((1ull << 32) + a.groups - 1) / a.groups));
+    a.window_log = 0;
+    while ((2 << a.window_log) * a.groups <= kWCap) ++a.window_log;
 }
 
-template <int VEC, int G, int WAVES, int U, bool SBUF>
+template <int VEC, int WAVES, int U, bool SBUF, bool HALVES = false>
 hipError_t run_rowblock(const RowblockArgs& args, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((csr_rowblock<VEC, G, WAVES, U, SBUF>), dim3(grid), dim3(WAVES * kWave), 0,
+    hipLaunchKernelGGL((csr_rowblock<VEC, WAVES, U, SBUF, HALVES>), dim3(grid), dim3(WAVES * kWave), 0,
                        stream, args);
     return hipGetLastError();
 }
 
-// Launch shapes: waves per workgroup (2, 4, 8) x entries in flight per lane
+// Launch shapes: waves per workgroup (2, 4, 8) x entries in flight per group
 // per step (4, 8).  B loads through a structured buffer unless B is too large
-// for one (then only the default shape, 8 waves x 4, is built).
-template <int VEC, int G>
+// for one (then only 8 waves x 4 is built).
+template <int VEC>
 hipError_t dispatch_shape(int waves, int unroll, bool sbuf, const RowblockArgs& args, int grid,
                           hipStream_t stream) {
-    if (!sbuf) return run_rowblock<VEC, G, 8, 4, false>(args, grid, stream);
+    if (!sbuf) return run_rowblock<VEC, 8, 4, false>(args, grid, stream);
     if (waves == 8) {
-        return unroll == 8 ? run_rowblock<VEC, G, 8, 8, true>(args, grid, stream)
-                           : run_rowblock<VEC, G, 8, 4, true>(args, grid, stream);
+        return unroll == 8 ? run_rowblock<VEC, 8, 8, true>(args, grid, stream)
+                           : run_rowblock<VEC, 8, 4, true>(args, grid, stream);
     }
     if (waves == 2) {
-        return unroll == 8 ? run_rowblock<VEC, G, 2, 8, true>(args, grid, stream)
-                           : run_rowblock<VEC, G, 2, 4, true>(args, grid, stream);
+        return unroll == 8 ? run_rowblock<VEC, 2, 8, true>(args, grid, stream)
+                           : run_rowblock<VEC, 2, 4, true>(args, grid, stream);
     }
-    return unroll == 8 ? run_rowblock<VEC, G, 4, 8, true>(args, grid, stream)
-                       : run_rowblock<VEC, G, 4, 4, true>(args, grid, stream);
+    return unroll == 8 ? run_rowblock<VEC, 4, 8, true>(args, grid, stream)
+                       : run_rowblock<VEC, 4, 4, true>(args, grid, stream);
 }
 
-template <int VEC>
-hipError_t dispatch_groups(int groups, int waves, int unroll, bool sbuf, const RowblockArgs& args,
-                           int grid, hipStream_t stream) {
-    if constexpr (VEC == 4) {
-        if (groups == 8) return dispatch_shape<VEC, 8>(waves, unroll, sbuf, args, grid, stream);
+template <bool HALVES>
+hipError_t dispatch_wide(int waves, const RowblockArgs& args, int grid, hipStream_t stream) {
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * kWave), 0, stream, args);
+        return hipGetLastError();
+    };
+    if constexpr (!HALVES) {
+        if (waves == 8) {
+            return args.groups == 1 ? run(csr_rowblock_wide<1, 8, false>)
+                                    : run(csr_rowblock_wide<2, 8, false>);
+        }
     }
-    if (groups == 4) return dispatch_shape<VEC, 4>(waves, unroll, sbuf, args, grid, stream);
-    if (groups == 2) return dispatch_shape<VEC, 2>(waves, unroll, sbuf, args, grid, stream);
-    return dispatch_shape<VEC, 1>(waves, unroll, sbuf, args, grid, stream);
+    return args.groups == 1 ? run(csr_rowblock_wide<1, 4, HALVES>)
+                            : run(csr_rowblock_wide<2, 4, HALVES>);
 }
 
-// Column slices for a K x N fp32 B: the fewest (a power of two, at most 8,
-// each slice at least 64 columns wide) that bring one XCD's share of B down
-// to its 4 MiB L2.  Measured on MI355X: B of 8 MiB (16384 x 128, 8192 x 256)
-// 1.2-1.7x faster with 2 slices; B of 4 MiB or less is fastest unsliced.
-int auto_slices(int K, int N) {
+// Column slices for a K x N fp32 B: the fewest (a power of two, at most 8) that
+// bring one XCD's share of B down to its 4 MiB L2, each at least 32 columns
+// wide (one 128-byte line of a B row); on rows of 16 entries and more, while
+// slices stay 64 columns wide, down to half of the L2, which A and C pass
+// through too.  Measured on MI355X over 70 uniform and power-law inputs with B
+// of 8 .. 256 MiB, against slices of at least 64 columns: 65536^2, 32 per row,
+// N = 256 252 -> 212 us; 32768^2, 32 per row, N = 128 46.7 -> 38.9 us; 8192^2, 100
+// per row, N = 512 70 -> 64 us.  B of 4 MiB or less is fastest unsliced.  Rows
+// that are no whole number of lines keep 64 columns: every slice of such a row
+// touches one line more (131072^2, 8 per row, N = 500: 414 us with 4 slices, 447
+// with 8).
+int auto_slices(int K, int N, double avg_row) {
     const long long b_bytes = static_cast<long long>(K) * N * 4;
+    if (b_bytes <= (4LL << 20)) return 1;
+    const int narrowest = N % 32 == 0 ? 32 : 64;
     int s = 1;
-    while (s < 8 && b_bytes > (4LL << 20) * s && N / (2 * s) >= 64) s *= 2;
+    while (s < 8 && ((b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest) ||
+                     (b_bytes > (2LL << 20) * s && N / (2 * s) >= 64 && avg_row >= 16.0))) {
+        s *= 2;
+    }
     return s;
 }
-
-int default_waves(int slices) { return slices == 1 ? 8 : 4; }
 
 // Waves of the engine resident at once on the chip: 16 per CU (four 4-wave
 // workgroups) on 256 CUs.
@@ -991,7 +1331,7 @@ int pow2_log_at_least(int x) {
 constexpr long kRowGroupTargetWaves = 8192;
 int row_group_lc_log(int M, int N, int vec) {
     int lc_log = pow2_log_at_least(ceil_div(N, vec));
-    while (lc_log > 4 && (static_cast<long>(M) << lc_log) / kWave >= 2 * kRowGroupTargetWaves) {
+    while (lc_log > 4 && N % 32 == 0 && (static_cast<long>(M) << lc_log) / kWave >= 2 * kRowGroupTargetWaves) {
         --lc_log;
     }
     return lc_log;
@@ -1007,8 +1347,9 @@ int row_group_lc_log(int M, int N, int vec) {
 int row_group_slices(int K, int N, double avg_row) {
     if (avg_row > 24.0) return 1;
     const long long b_bytes = static_cast<long long>(K) * N * 4;
+    const int narrowest = N % 32 == 0 ? 32 : 64;  // whole lines, as in auto_slices
     int s = 1;
-    while (s < 8 && b_bytes > (4LL << 20) * s && N / (2 * s) >= 32) s *= 2;
+    while (s < 8 && b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest) s *= 2;
     return s;
 }
 
@@ -1202,61 +1543,73 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
         }
         return launch_row_groups(A, B, C, N, stream, vec, o);
     }
+    const double avg = A.nnz > 0 ? static_cast<double>(A.nnz) / M : 1.0;
     // Column slices (XCD-aware, see the kernel): 1, 2, 4 or 8.
     int slices = o.slices;
-    if (slices == 0) slices = role == CsrRole::Tiled ? 1 : auto_slices(A.num_cols, N);
+    if (slices == 0) slices = role == CsrRole::Tiled ? 1 : auto_slices(A.num_cols, N, avg);
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     int slice_cols = ceil_div(N, slices);
     slice_cols = ceil_div(slice_cols, vec) * vec;
-    const int groups = pick_groups(slice_cols, vec, want_groups);
-    // Defaults measured on MI355X (c1 / c2 / c5 and uniform / power-law
-    // sweeps): 8 waves per workgroup without column slices (a workgroup's
-    // nonzeros are split over its waves, so a long row is shared by eight),
-    // 4 with them (the sliced launch has twice the workgroups per row block),
-    // 4 entries per group in flight per step (two steps in flight), about 160
-    // nonzeros per wave and at least 512 workgroups (two per CU) when the
-    // matrix allows it: many small workgroups keep skewed rows balanced.
-    // Rows known to be even (max_row_hint): the whole-round grid of 4-wave
-    // workgroups.
-    const bool even = split == nullptr && bounds == nullptr && o.rows_per_block <= 0 &&
-                      rows_even(M, A.nnz, o.max_row_hint);
-    const int waves = (o.waves == 2 || o.waves == 4 || o.waves == 8) ? o.waves
-                      : even                                         ? 4
-                                                                     : default_waves(slices);
+    // Defaults measured on MI355X (uniform and power-law sweeps): 8 waves per
+    // workgroup without column slices (a workgroup's nonzeros are split over
+    // its waves, so a long row is shared by eight: power-law 2048^2, N = 128 9.5
+    // us with 8, 12.1 with 4), 4 with them (more workgroups per row block) and
+    // on merge-path parts; 4 rows in flight per group; about 160 nonzeros per
+    // wave and at least 512 row blocks (256 with slices) when the matrix allows
+    // it: many small workgroups keep skewed rows balanced.  Rows known to be
+    // even (max_row_hint): the whole-round grid of 4-wave workgroups.
     const int unroll = o.unroll == 8 ? 8 : 4;
     const bool sbuf = o.global_loads == 0 && b_fits_buffer(A.num_cols, N);
 
-    RowblockArgs args{A.row_ptr, A.col_idx, A.values, B,       C,       bounds, M, N, A.num_cols,
-                      0,         0,         slices,   slice_cols, nullptr, nullptr, 0};
+    RowblockArgs args{};
+    RowblockPart& part = args.part;
+    part = RowblockPart{A.row_ptr, A.col_idx, A.values, B, C};
+    part.K          = A.num_cols;
+    args.M          = M;
+    args.N          = N;
+    args.slices     = slices;
+    args.slice_cols = slice_cols;
+    set_groups(args, slice_cols, vec, want_groups);
+    // The whole-round grid is for few groups: it leaves more of them too few
+    // row pieces each (65536^2, 40 per row, N = 256, eight slices of four groups:
+    // 305 us with it, 260 without).
+    const bool even = split == nullptr && bounds == nullptr && o.rows_per_block <= 0 &&
+                      args.groups <= 2 && rows_even(M, A.nnz, o.max_row_hint);
+    const int waves = (o.waves == 2 || o.waves == 4 || o.waves == 8) ? o.waves
+                      : even || slices > 1 || split != nullptr       ? 4
+                                                                     : 8;
     if (split != nullptr) {
-        args.bounds     = nullptr;
-        args.split_rows = split->rows;
-        args.carry      = split->carry;
-        args.nnz        = A.nnz;
-        args.nblocks    = split->parts;
+        part.split_rows = split->rows;
+        part.carry      = split->carry;
+        part.nnz        = A.nnz;
+        part.nblocks    = split->parts;
     } else if (bounds != nullptr) {
-        args.nblocks = parts;
+        args.bounds  = bounds;
+        part.nblocks = parts;
     } else {
         int rpb = o.rows_per_block;
         if (rpb <= 0 && even) {
             rpb = round_rows_per_block(M, A.nnz, slices, waves);
         } else if (rpb <= 0) {
-            const double avg = A.nnz > 0 ? static_cast<double>(A.nnz) / M : 1.0;
             rpb = static_cast<int>(160.0 * waves / std::max(avg, 1.0) + 0.5);
-            rpb = std::min(rpb, M / 512);
+            rpb = std::min(rpb, M / (slices == 1 ? 512 : 256));
         }
         rpb = std::max(1, std::min(rpb, kRpCap));
         args.rows_per_block = rpb;
-        args.nblocks = ceil_div(M, rpb);
+        part.nblocks = ceil_div(M, rpb);
     }
-    const int grid = slices == 1 ? args.nblocks : ceil_div(args.nblocks, 8 / slices) * 8;
+    const int grid = slices == 1 ? part.nblocks : ceil_div(part.nblocks, 8 / slices) * 8;
     hipError_t e;
-    if (vec == 4) {
-        e = dispatch_groups<4>(groups, waves, unroll, sbuf, args, grid, stream);
+    const bool balanced = even || split != nullptr;
+    if (balanced && sbuf && vec == 4 && args.groups <= 2 && o.groups == 0 && o.waves == 0 &&
+        o.unroll == 0) {
+        e = dispatch_wide<false>(even || slices > 1 ? 4 : 8, args, grid, stream);
+    } else if (vec == 4) {
+        e = dispatch_shape<4>(waves, unroll, sbuf, args, grid, stream);
     } else if (vec == 2) {
-        e = dispatch_groups<2>(groups, waves, unroll, sbuf, args, grid, stream);
+        e = dispatch_shape<2>(waves, unroll, sbuf, args, grid, stream);
     } else {
-        e = dispatch_groups<1>(groups, waves, unroll, sbuf, args, grid, stream);
+        e = dispatch_shape<1>(waves, unroll, sbuf, args, grid, stream);
     }
     if (e == hipSuccess && split != nullptr) {
         hipLaunchKernelGGL(csr_split_fixup, dim3(split->parts), dim3(64), 0, stream, A.row_ptr,
@@ -1315,9 +1668,25 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     const int slices = row_group_slices(K, N, avg_row);
     const int lc     = 1 << row_group_lc_log(M, ceil_div(ceil_div(N, slices), vec) * vec, vec);
     if (max_row > std::max(16384.0 / lc, 8.0 * avg_row)) return false;
+    // A B past the L2s whose rows are whole lines: the engine's slices of 32
+    // columns beat the row groups on longer rows (65536^2, 40 per row, N = 64 61
+    // against 72 us, N = 128 120 against 155 us; 32768^2, 40 per row, N = 256 94
+    // against 131 us) and at any length once B is far larger.  Other widths
+    // cannot be cut that narrow, and there the row groups win on even rows
+    // (24576^2, 100 per row, N = 100 65 against 99 us; over 90 inputs with N = 33
+    // .. 250 they lose at most 3%, and at N = 250 on rows of 24 and fewer 15%).
+    const double b_mib = static_cast<double>(K) * N / (1 << 18);
+    const bool lines = N % 32 == 0;
+    if (N <= 32 && K > 98304 && avg_row >= 16.0) return false;
+    if (lines && N > 32 && N <= 64 && b_mib >= 16.0) return false;
+    if (lines && N > 64 && b_mib > 4.0 &&
+        (avg_row >= (N > 128 ? 16.0 : 24.0) || (N <= 128 && b_mib >= 32.0))) {
+        return false;
+    }
     if (N <= 64) return M >= 2048 || avg_row <= 100.0;
     if (N * avg_row <= 2048.0 || (N <= 256 && slices > 1)) return true;
     if (max_row > 2.0 * avg_row + 32.0) return false;  // uneven rows
+    if (!lines && N <= 256 && b_mib > 4.0) return true;
     if (N * avg_row <= 4096.0) return true;
     if (N > 128) return false;
     if (M > 4096 && M <= 8192 && avg_row >= 64.0) return false;
@@ -1369,21 +1738,25 @@ Error launch_csr_khalf(const KHalfPlan& p, const float* B, float* C, hipStream_t
         }
     }
     const int N = p.N;
-    RowblockArgs args{p.half[0].row_ptr, p.half[0].col_idx, p.half[0].values, B, C, nullptr,
-                      p.M, N, p.K0, 0, p.parts[0], 1, N, p.rows[0], p.carry[0], p.half[0].nnz};
-    args.halves      = 1;
-    args.row_ptr1    = p.half[1].row_ptr;
-    args.col_idx1    = p.half[1].col_idx;
-    args.vals1       = p.half[1].values;
-    args.B1          = B + static_cast<size_t>(p.K0) * N;
-    args.C1          = p.partial;
-    args.K1          = p.K - p.K0;
-    args.split_rows1 = p.rows[1];
-    args.carry1      = p.carry[1];
-    args.nnz1        = p.half[1].nnz;
-    args.nblocks1    = p.parts[1];
+    RowblockArgs args{};
+    for (int h = 0; h < 2; ++h) {
+        RowblockPart& part = h == 0 ? args.part : args.upper;
+        part = RowblockPart{p.half[h].row_ptr, p.half[h].col_idx, p.half[h].values,
+                            h == 0 ? B : B + static_cast<size_t>(p.K0) * N,
+                            h == 0 ? C : p.partial};
+        part.split_rows = p.rows[h];
+        part.carry      = p.carry[h];
+        part.nnz        = p.half[h].nnz;
+        part.K          = h == 0 ? p.K0 : p.K - p.K0;
+        part.nblocks    = p.parts[h];
+    }
+    args.M          = p.M;
+    args.N          = N;
+    args.slice_cols = N;
+    set_groups(args, N, 4, 0);
     const int grid   = 8 * ceil_div(std::max(p.parts[0], p.parts[1]), 4);
-    hipError_t e = dispatch_groups<4>(pick_groups(N, 4, 0), 4, 4, true, args, grid, stream);
+    hipError_t e = args.groups <= 2 ? dispatch_wide<true>(4, args, grid, stream)
+                                    : run_rowblock<4, 4, 4, true, true>(args, grid, stream);
     if (e == hipSuccess) {
         const long long chunks = static_cast<long long>(p.M) * N / 4;
         hipLaunchKernelGGL(csr_khalf_fixup, dim3(static_cast<unsigned>((chunks + 255) / 256)),
