@@ -1,10 +1,10 @@
 // CSR x dense kernels for gfx950 (wave64, 256 CUs in 8 XCDs).
 //
-//   csr_lane_per_output   role of spmm_baseline   (spmm_baseline.cu:11-25)
-//   csr_wave_per_row      role of spmm_memopt/_v2 (spmm_memopt.cu:11-38)
-//   csr_rowblock          role of spmm_tiled*     (spmm_tiled_v3.cu:21-104), the engine
+//   csr_rows_in_order  role of spmm_baseline and spmm_memopt/_v2
+//                      (spmm_baseline.cu:11-25, spmm_memopt.cu:11-38)
+//   csr_rowblock       role of spmm_tiled* (spmm_tiled_v3.cu:21-104), the engine
 //
-// All three accumulate in fp32 with fused multiply-adds.  C is fully written
+// All accumulate in fp32 with fused multiply-adds.  C is fully written
 // (rows without nonzeros get zeros), so callers never clear it.
 
 #include <hip/hip_runtime.h>
@@ -57,62 +57,6 @@ template <> struct Vec<4> {
 template <int VEC>
 __device__ __forceinline__ typename Vec<VEC>::T vzero() {
     return typename Vec<VEC>::T(0.0f);
-}
-
-// ---------------------------------------------------------------------------
-// Role: spmm_baseline.  One lane per C(i, j); a wave spans 64 columns of one
-// row, so the row's (col, value) reads are wave-uniform and the B reads are
-// one coalesced 256-byte segment per nonzero.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void csr_lane_per_output(
-    int M, int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
-    const float* __restrict__ vals, const float* __restrict__ B, float* __restrict__ C) {
-    const int j = blockIdx.x * kWave + threadIdx.x;
-    const int i = blockIdx.y * 4 + threadIdx.y;
-    if (i >= M || j >= N) return;
-    const int p0 = row_ptr[i];
-    const int p1 = row_ptr[i + 1];
-    float sum = 0.f;
-    for (int p = p0; p < p1; ++p) {
-        sum = __builtin_fmaf(vals[p], B[static_cast<size_t>(col_idx[p]) * N + j], sum);
-    }
-    C[static_cast<size_t>(i) * N + j] = sum;
-}
-
-// ---------------------------------------------------------------------------
-// Role: spmm_memopt / spmm_memopt_v2.  One wave per row; lane l owns columns
-// c0 + l + 64*t (t < CPL) of each column pass, every nonzero is read once per
-// pass with a wave-uniform (scalar) load.
-// ---------------------------------------------------------------------------
-template <int CPL, int MIN_WAVES_PER_EU>
-__global__ __launch_bounds__(256, MIN_WAVES_PER_EU) void csr_wave_per_row(
-    int M, int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
-    const float* __restrict__ vals, const float* __restrict__ B, float* __restrict__ C) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & (kWave - 1);
-    if (row >= M) return;
-    const int p0 = row_ptr[row];
-    const int p1 = row_ptr[row + 1];
-    float* crow = C + static_cast<size_t>(row) * N;
-    for (int c0 = 0; c0 < N; c0 += kWave * CPL) {
-        float acc[CPL];
-#pragma unroll
-        for (int t = 0; t < CPL; ++t) acc[t] = 0.f;
-        for (int p = p0; p < p1; ++p) {
-            const float v = vals[p];
-            const float* brow = B + static_cast<size_t>(col_idx[p]) * N;
-#pragma unroll
-            for (int t = 0; t < CPL; ++t) {
-                const int c = c0 + lane + kWave * t;
-                if (c < N) acc[t] = __builtin_fmaf(v, brow[c], acc[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < CPL; ++t) {
-            const int c = c0 + lane + kWave * t;
-            if (c < N) crow[c] = acc[t];
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -256,6 +200,106 @@ __device__ __forceinline__ int lane_col(int col, int cend) {
 }
 
 __device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m); }
+
+template <int VEC>
+__device__ __forceinline__ typename Vec<VEC>::T fma_vec(float v, typename Vec<VEC>::T b,
+                                                        typename Vec<VEC>::T acc) {
+    if constexpr (VEC == 1) {
+        return __builtin_fmaf(v, b, acc);
+    } else {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) acc[i] = __builtin_fmaf(v, b[i], acc[i]);
+        return acc;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Role: spmm_baseline, spmm_memopt, spmm_memopt_v2: every output is one chain of
+// fused multiply-adds in the row's order, the reference kernels' bits.
+//
+// The chain leaves the columns and the rows to run in parallel and, inside a
+// row, the loads: L column lanes of VEC floats own a row (64 / L rows per wave),
+// U entries' B segments are in flight while the chain takes them in order.  The
+// group loads L column indices and values at a time, one each per lane, and
+// hands them out by readlane (L = 64: one row per wave, so the B row's address
+// is scalar) or shuffle; groups of under eight lanes load them directly.
+// Latency bounds it: U x resident waves loads in flight.  Measured on MI355X
+// against one wave per row with 4-byte lanes and one entry at a time: 4096^2, 41
+// per row, N = 256 64.9 -> 10.4 us (2.6 -> 16.5 TB/s of gathered rows), N = 128 22.5 ->
+// 6.8 us; 65536^2, 16 per row, N = 1 44.5 -> 8.3 us; and against one lane per output
+// (spmm_baseline before) 24.5 -> 10.4, 14.6 -> 6.8 and 39.0 -> 8.3 us.
+// ---------------------------------------------------------------------------
+enum class Hand { Direct, Shuffle, Readlane };
+
+template <int VEC, Hand HAND>
+__global__ __launch_bounds__(256) void csr_rows_in_order(
+    int M, int N, int lc_log, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
+    const float* __restrict__ vals, const float* __restrict__ B, float* __restrict__ C) {
+    using VT = typename Vec<VEC>::T;
+    using MT = typename Vec<VEC>::Mem;
+    constexpr int U = HAND == Hand::Readlane ? 16 : 8;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int L    = HAND == Hand::Readlane ? kWave : 1 << lc_log;
+    const int gl   = lane & (L - 1);
+    const int row  = (blockIdx.x * 4 + wave) * (kWave / L) +
+                    (HAND == Hand::Readlane ? 0 : lane >> lc_log);
+    if (row >= M) return;  // whole groups, and no barrier follows
+    const int p0 = row_ptr[row];
+    const int p1 = row_ptr[row + 1];
+    float* crow = C + static_cast<size_t>(row) * N;
+    for (int n0 = blockIdx.y * (L * VEC); n0 < N; n0 += gridDim.y * (L * VEC)) {
+        const int    col  = lane_col<VEC>(n0 + gl * VEC, N);
+        const float* bcol = B + col;
+        VT acc = vzero<VEC>();
+        // Entries [p, p + cnt) of the chain, cnt <= L, U at a time; entry j is
+        // handed out by take(j).
+        auto chain = [&](int cnt, auto take) {
+            for (int j0 = 0; j0 < cnt; j0 += U) {
+                VT    b[U];
+                float v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    int k;
+                    take(min(j0 + u, cnt - 1), k, v[u]);
+                    b[u] = *reinterpret_cast<const MT*>(bcol + static_cast<size_t>(k) * N);
+                }
+                if (j0 + U <= cnt) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc = fma_vec<VEC>(v[u], b[u], acc);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (j0 + u < cnt) acc = fma_vec<VEC>(v[u], b[u], acc);
+                    }
+                }
+            }
+        };
+        if constexpr (HAND == Hand::Direct) {
+            chain(p1 - p0, [&](int j, int& k, float& v) {
+                k = col_idx[p0 + j];
+                v = vals[p0 + j];
+            });
+        } else {
+            for (int p = p0; p < p1; p += L) {
+                const int   q  = min(p + gl, p1 - 1);
+                const int   kc = col_idx[q];
+                const float vc = vals[q];
+                chain(min(L, p1 - p), [&](int j, int& k, float& v) {
+                    if constexpr (HAND == Hand::Readlane) {
+                        k = __builtin_amdgcn_readlane(kc, j);
+                        v = __builtin_bit_cast(
+                            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vc), j));
+                    } else {
+                        k = __shfl(kc, (lane & ~(L - 1)) + j);
+                        v = __shfl(vc, (lane & ~(L - 1)) + j);
+                    }
+                });
+            }
+        }
+        if (n0 + gl * VEC < N) store_vec<VEC>(crow + col, acc);
+    }
+}
 
 // Orders a wave's LDS writes before its own lanes' reads of them.
 __device__ __forceinline__ void wave_lds_sync() {
@@ -1447,6 +1491,25 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
     return from_hip(e, "csr row groups launch");
 }
 
+// Column lanes: the fewest (a power of two, at most 64) that cover N; wider N in
+// column tiles of 256, a workgroup each.
+Error launch_in_order(const CSR& A, const float* B, float* C, int N, hipStream_t stream) {
+    const int vec    = pick_vec(N, 0);
+    const int lc_log = pow2_log_at_least(ceil_div(N, vec));
+    const dim3 grid(ceil_div(A.num_rows, 4 * (kWave >> lc_log)),
+                    std::min(ceil_div(N, vec << lc_log), 65535));
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, A.num_rows, N, lc_log, A.row_ptr,
+                           A.col_idx, A.values, B, C);
+        return from_hip(hipGetLastError(), "csr in-order launch");
+    };
+    if (vec == 1) return run(csr_rows_in_order<1, Hand::Direct>);
+    if (vec == 2) return run(csr_rows_in_order<2, Hand::Direct>);
+    if (lc_log == 6) return run(csr_rows_in_order<4, Hand::Readlane>);
+    return lc_log >= 3 ? run(csr_rows_in_order<4, Hand::Shuffle>)
+                       : run(csr_rows_in_order<4, Hand::Direct>);
+}
+
 Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int N,
                       hipStream_t stream, const int* bounds, int parts, const EngineOpts* opts,
                       const SplitPlan* split) {
@@ -1463,24 +1526,8 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     if (bounds != nullptr && parts < 1) return fail(kInvalid, "partition needs parts >= 1");
 
     const int M = A.num_rows;
-    switch (role) {
-        case CsrRole::Baseline: {
-            dim3 block(kWave, 4);
-            dim3 grid(ceil_div(N, kWave), ceil_div(M, 4));
-            hipLaunchKernelGGL(csr_lane_per_output, grid, block, 0, stream, M, N, A.row_ptr,
-                               A.col_idx, A.values, B, C);
-            return from_hip(hipGetLastError(), "spmm_baseline launch");
-        }
-        case CsrRole::Memopt:
-            hipLaunchKernelGGL((csr_wave_per_row<2, 1>), dim3(ceil_div(M, 4)), dim3(256), 0, stream,
-                               M, N, A.row_ptr, A.col_idx, A.values, B, C);
-            return from_hip(hipGetLastError(), "spmm_memopt launch");
-        case CsrRole::MemoptV2:
-            hipLaunchKernelGGL((csr_wave_per_row<2, 8>), dim3(ceil_div(M, 4)), dim3(256), 0, stream,
-                               M, N, A.row_ptr, A.col_idx, A.values, B, C);
-            return from_hip(hipGetLastError(), "spmm_memopt_v2 launch");
-        default:
-            break;
+    if (role == CsrRole::Baseline || role == CsrRole::Memopt || role == CsrRole::MemoptV2) {
+        return launch_in_order(A, B, C, N, stream);
     }
 
     EngineOpts o = opts ? *opts : EngineOpts{};

@@ -550,7 +550,9 @@ def test_any_width_and_alignment(S, O, torch, N, shift):
     rows = torch.from_numpy(S.nnz_split_rows(A, parts)).cuda()
     bounds = torch.from_numpy(S.nnz_balanced_bounds(A, parts)).cuda()
     E = S.EngineOptsT
-    runs = {"tiled": lambda C: S.spmm_csr("tiled", dA, dB, C),
+    runs = {"baseline": lambda C: S.spmm_csr("baseline", dA, dB, C),
+            "memopt": lambda C: S.spmm_csr("memopt", dA, dB, C),
+            "tiled": lambda C: S.spmm_csr("tiled", dA, dB, C),
             "tiled_v3": lambda C: S.spmm_csr("tiled_v3", dA, dB, C),
             "engine": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(0, 4), C),
             "slices": lambda C: S.spmm_tiled_v3_opts(dA, dB, E(0, 0, 0, 0, 0, 4), C),
