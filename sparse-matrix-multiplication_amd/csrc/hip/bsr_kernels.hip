@@ -110,11 +110,16 @@ __device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int& bx, int& by)
 
 
 // ---------------------------------------------------------------------------
-// Wave kernel (the default path): one wave = one block-row x 16*J columns,
-// four independent waves per workgroup, no workgroup barriers.  Maximum
-// parallelism and a small LDS footprint (one 32 x (16J+16) fp16 tile per
-// wave) keep many waves resident, which is what hides the latency of the
-// short dependent chain row_ptr -> col_idx -> (A, B) -> MFMA.
+// Wave kernel (pointer addressing: what the record kernel below does not take):
+// one wave = one block-row x 16*J columns, four independent waves per
+// workgroup, no workgroup barriers.  Maximum parallelism and a small LDS
+// footprint (one 32 x (16J+16) fp16 tile per wave) keep many waves resident,
+// which is what hides the latency of the short dependent chain row_ptr ->
+// col_idx -> (A, B) -> MFMA.  Latency and the B re-reads of every block-row
+// bound it.  Rows of B may start at any element: 16-byte chunks at any N and
+// alignment (MI355X against one load per element, which bound those widths
+// before: 5003 x 6997 blocks at 15%, N = 100 66.2 -> 15.1 us; 8192^2 at 12.5%, N =
+// 500 228 -> 46 us).
 //   - The block-row's block-columns come in with one vector load (lane i
 //     holds col_idx[first + i], 64 per chunk) and are broadcast with
 //     v_readlane, so pairs need no further index loads.
@@ -125,6 +130,15 @@ __device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int& bx, int& by)
 // LDS accesses of one wave execute in program order, so the single tile
 // needs no barrier between a pair's reads and the next pair's writes.
 // ---------------------------------------------------------------------------
+// Eight fp16 at any element address (a 16-byte global load needs no alignment).
+typedef f16x8 Mem __attribute__((aligned(2)));
+
+// The 8 - n upper elements of v moved down, zeros above them.
+__device__ __forceinline__ f16x8 drop_low(f16x8 v, int n) {
+    unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v);
+    return __builtin_bit_cast(f16x8, n < 8 ? x >> (16 * n) : static_cast<unsigned __int128>(0));
+}
+
 template <int J, int D, bool VEC>
 __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
     constexpr int NT  = 16 * J;          // columns per wave
@@ -159,6 +173,7 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
     struct PairRegs {
         f16x8 b[CPL];
         f16x8 af;
+        int   shift[CPL];  // elements the chunk was loaded before its own first
         bool  b_ok[CPL];
         bool  a_ok;
     };
@@ -178,10 +193,19 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
             const bool ok = (s < 16 || two) && k < a.K && n < a.N;
             r.b_ok[c] = ok;
             if constexpr (VEC) {
+                // A row may start at any element (Mem) and the last chunk of a
+                // row may run into the next row: those products land in output
+                // columns >= N, which are never stored.  Only past the end of
+                // B is the chunk taken from B's last 8 elements instead and
+                // shifted into place when it is used -- no branch here, so the
+                // loads of all pairs in flight stay independent.
                 const size_t off = ok ? static_cast<size_t>(k) * a.N + n : 0;
-                r.b[c] = *reinterpret_cast<const f16x8*>(a.B + off);
+                const size_t at  = min(off, static_cast<size_t>(a.K) * a.N - 8);
+                r.shift[c] = static_cast<int>(off - at);
+                r.b[c] = *reinterpret_cast<const Mem*>(a.B + at);
             } else {
                 const size_t row = ok ? static_cast<size_t>(k) * a.N : 0;
+                r.shift[c] = 0;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const bool in = ok && n + e < a.N;
@@ -201,8 +225,12 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
         for (int c = 0; c < CPL; ++c) {
             const int idx = lane + c * 64;
             const f16x8 zero = f16x8(static_cast<_Float16>(0.0f));
+            f16x8 b = r.b[c];
+            if constexpr (VEC) {
+                if (__builtin_expect(__any(r.shift[c] != 0), 0)) b = drop_low(b, r.shift[c]);
+            }
             *reinterpret_cast<f16x8*>(&tile[(idx / CH) * S + (idx % CH) * 8]) =
-                r.b_ok[c] ? r.b[c] : zero;
+                r.b_ok[c] ? b : zero;
         }
         const f16x8 af = r.a_ok ? r.af : f16x8(static_cast<_Float16>(0.0f));
         const _Float16* rowp = &tile[(8 * g + (t >> 2)) * S + 4 * (t & 3)];
@@ -970,10 +998,13 @@ hipError_t run_wave(BsrArgs args, hipStream_t stream, bool pointer_addressing) {
                            args);
         return hipGetLastError();
     }
-    if (args.b_vec_ok) {
+    if (static_cast<long long>(args.K) * args.N >= 8) {
         hipLaunchKernelGGL((bsr_wave_kernel<J, D, true>), grid, dim3(256), 0, stream, args);
-    } else {
-        hipLaunchKernelGGL((bsr_wave_kernel<J, D, false>), grid, dim3(256), 0, stream, args);
+    } else {  // B is smaller than one chunk
+        args.tiles_n  = 1;
+        args.wg_total = ceil_div(args.block_rows, 4);
+        hipLaunchKernelGGL((bsr_wave_kernel<1, 1, false>), dim3(args.wg_total), dim3(256), 0,
+                           stream, args);
     }
     return hipGetLastError();
 }
@@ -1113,14 +1144,20 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
     // then the extra waves of two tiles hide more latency (e.g. uniform
     // 8192^2 density 0.01 N=128: 67 -> 48 us).  Four pairs in flight pay on
     // long block-rows: >= 30 blocks at two tiles, >= 96 at four (uniform
-    // 4096^2 density 0.01 N=128: 26.4 -> 20.3 us).  The pointer-arithmetic
-    // form keeps two tiles and two pairs: it has no buffer-to-LDS staging,
-    // and four tiles measured slower there.
+    // 4096^2 density 0.01 N=128: 26.4 -> 20.3 us).  The pointer-arithmetic form
+    // (widths that are no multiple of 8, B off 16 bytes, buffers past 2 GiB)
+    // stages through registers: four tiles pay from 2048 waves on, with one
+    // pair in flight (8192^2 blocks at 12.5%, N = 500: 46 us against 75 with two
+    // tiles and 52 with two pairs; at 1024 waves 52 against 35), and one tile
+    // below 512 waves of two (2000^2, N = 36: 4.1 against 5.1 us).
     const long waves4 = static_cast<long>(A.block_rows) * ((N + 63) / 64);
+    const long waves2 = static_cast<long>(A.block_rows) * ((N + 31) / 32);
     const int j_auto =
-        N <= 16 ? 1 : ((rec && waves4 >= 1024 && (bpr >= 12.0 || waves4 >= 2048)) ? 4 : 2);
+        N <= 16 ? 1
+        : rec   ? ((waves4 >= 1024 && (bpr >= 12.0 || waves4 >= 2048)) ? 4 : 2)
+                : (waves4 >= 2048 ? 4 : (waves2 >= 512 ? 2 : 1));
     const int j = (o.tiles == 1 || o.tiles == 2 || o.tiles == 4) ? o.tiles : j_auto;
-    const int d_auto = (rec && bpr >= (j == 4 ? 96.0 : 30.0)) ? 4 : 2;
+    const int d_auto = rec ? (bpr >= (j == 4 ? 96.0 : 30.0) ? 4 : 2) : (j == 4 ? 1 : 2);
     const int d = (o.depth == 1 || o.depth == 2 || o.depth == 4) ? o.depth : d_auto;
     const bool ptr = o.addressing == 1;
     e = j == 1 ? dispatch_wave<1>(d, ptr, args, stream)

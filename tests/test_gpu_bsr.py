@@ -403,3 +403,32 @@ def test_wmma_linearity_c4(S, O, torch):
     c1 = S.spmm_wmma(dA, B16)
     c2 = S.spmm_wmma(dA, B16 * 2)
     assert torch.equal(c2, c1 * 2)
+
+
+@pytest.mark.parametrize("N", [1, 3, 7, 9, 20, 33, 50, 63, 100, 129, 200])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_wmma_any_width_and_alignment(S, O, torch, N, shift):
+    # 16-byte chunks of B rows that start at any fp16 element, the last chunk
+    # of a row running into the next row and, at B's end, taken from before it.
+    # B and C start `shift` elements past an aligned address inside buffers
+    # whose other elements are NaN: a read outside B would show in C (every
+    # column of the last block-column's rows is multiplied), a write outside C
+    # would change a NaN.  K = 1 with N < 8 is smaller than one chunk.
+    for M, K, dens in ((70, 150, 0.2), (33, 47, 1.0), (40, 1, 1.0)):
+        A = S.generate_uniform_random_csr(M, K, dens, 7 + N)
+        A.values = S.round_to_fp16(A.values)
+        B = S.round_to_fp16(np.random.default_rng(N).uniform(-1, 1, (K, N)).astype(np.float32))
+        hb, B16, C32, C64, absC = _refs(S, O, A, B)
+        bbuf = torch.full((K * N + 16,), float("nan"), dtype=torch.float16, device="cuda")
+        dB = bbuf[8 + shift:8 + shift + K * N].view(K, N)
+        dB.copy_(torch.from_numpy(B16.view(np.float16)))
+        for tiles, depth in ((0, 0), (1, 1), (2, 2), (4, 4)):
+            cbuf = torch.full((M * N + 8,), float("nan"), device="cuda")
+            dC = cbuf[4 + shift:4 + shift + M * N].view(M, N)
+            say(f"wmma any width M={M} K={K} N={N} shift={shift} tiles={tiles} depth={depth}")
+            S.spmm_wmma_opts(S.DeviceBSR(hb), dB, S.BsrOptsT(tiles=tiles, depth=depth), dC)
+            torch.cuda.synchronize()
+            check_bsr(dC.cpu().numpy(), C32, absC)
+            check_csr(dC.cpu().numpy(), C64, absC, tol=1e-5)
+            assert torch.isnan(cbuf[:4 + shift]).all()
+            assert torch.isnan(cbuf[4 + shift + M * N:]).all()
