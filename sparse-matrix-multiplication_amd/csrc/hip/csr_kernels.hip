@@ -1425,11 +1425,17 @@ hipError_t run_row_groups(const RowGroupArgs& args, bool coop, bool long_rows, i
 //  - column lanes cover N in one pass (up to 64 lanes), except that 32 or 64
 //    column lanes drop to 16 (two or four passes) while the matrix would
 //    still give >= 16384 waves (e.g. M = 32768, N = 128: 96 -> 89 us);
-//  - entry lanes ~1.5 * sqrt(average row) as a power of two, but no more than
-//    keep the grid near 8192 waves (32 per CU): beyond that, more rows per
-//    wave beat more lanes per row;
-//  - 4 entries per entry lane per iteration from 32 entries per row on while
-//    B is at most 2 MiB (latency-bound: few, long rows), else 2 -- with B
+//  - entry lanes ~1.5 * sqrt(average row) as a power of two (sqrt from 4 column
+//    lanes on), but on rows of under 20 entries, or from 16 column lanes on, no
+//    more than keep the grid near 8192 waves (32 per CU): beyond that, more
+//    rows per wave beat more lanes per row.  Longer rows of narrow B are bound
+//    by one 128-byte line per entry into the L1s (262144 rows of 24, N = 1: 6.3 M
+//    lines in 31 us, 26 TB/s, where gathers saturate), and a lane that walks a
+//    row alone also takes a line of col_idx and of values per step: 45 -> 31 us
+//    there, 131072 rows of 120, N = 8 168 -> 96 us; of 3 at N = 32 12.3 against 13.4
+//    with two lanes instead of one;
+//  - 4 entries per entry lane per iteration on those, and from 32 entries per
+//    row on while B is at most 2 MiB (latency-bound: few, long rows), else 2 -- with B
 //    beyond one XCD's L2, fewer gathers in flight keep more of it cached
 //    (M = 32768, N = 128, 82 entries per row: 123 -> 88 us);
 //  - the cooperative loads (one column/value load per L entries, handed out
@@ -1450,6 +1456,7 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     const int slice_cols = ceil_div(ceil_div(N, slices), vec) * vec;
     const int lc_log = row_group_lc_log(M, slice_cols, vec);
+    const bool deep = avg >= 20.0 && lc_log <= 3;
     int le_log;
     if (o.entry_lanes != 0) {
         if (o.entry_lanes < 0 || o.entry_lanes > 64 || (o.entry_lanes & (o.entry_lanes - 1)) != 0) {
@@ -1457,18 +1464,20 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
         }
         le_log = pow2_log_at_least(o.entry_lanes);
     } else {
-        const double want = 1.5 * std::sqrt(std::max(avg, 1.0));
+        const double want = (deep && lc_log >= 2 ? 1.0 : 1.5) * std::sqrt(std::max(avg, 1.0));
         le_log = static_cast<int>(std::lround(std::log2(want)));
-        const long cap =
-            kTargetWaves * kWave / std::max(1L, (static_cast<long>(M) << lc_log) * slices);
-        int cap_log = 0;
-        while ((2L << cap_log) <= cap) ++cap_log;
-        le_log = std::min(le_log, cap_log);
+        if (!deep) {
+            const long cap =
+                kTargetWaves * kWave / std::max(1L, (static_cast<long>(M) << lc_log) * slices);
+            int cap_log = 0;
+            while ((2L << cap_log) <= cap) ++cap_log;
+            le_log = std::min(le_log, cap_log);
+        }
     }
     le_log = std::max(0, std::min(le_log, 6 - lc_log));
     const bool b_small = static_cast<long long>(A.num_cols) * N * 4 <= (2LL << 20);
     const int unroll = (o.unroll == 2 || o.unroll == 4) ? o.unroll
-                                                        : ((avg >= 32.0 && b_small) ? 4 : 2);
+                                                        : (deep || (avg >= 32.0 && b_small) ? 4 : 2);
     bool coop;
     if (o.row_groups == 2) coop = false;
     else if (o.row_groups == 3) coop = true;

@@ -571,3 +571,24 @@ def test_any_width_and_alignment(S, O, torch, N, shift):
         torch.cuda.synchronize()
         check_csr(dC.cpu().numpy(), C64, absC)
         assert torch.isnan(cbuf[:4 + shift]).all() and torch.isnan(cbuf[4 + shift + dC.numel():]).all()
+
+
+@pytest.mark.parametrize("N", [1, 3, 4, 8, 13, 16, 29, 32])
+def test_row_groups_many_rows(S, O, torch, N):
+    # More rows than the lane cap of short rows leaves entry lanes for: rows
+    # average 20 entries and more, with empty rows and rows of more entries
+    # than a group takes itself.
+    for mean, longest in ((24.0, 400), (70.0, 3000)):
+        A = S.generate_power_law_csr(66001, 3001, mean, 1.5, longest, 17)
+        B = np.random.default_rng(N).uniform(-1, 1, (A.num_cols, N)).astype(np.float32)
+        C64, absC = O.csr_spmm_f64(A.row_ptr, A.col_idx, A.values, B)
+        dA, dB = S.DeviceCSR(A), torch.from_numpy(B).cuda()
+        for name, opts in (("default", None), ("groups", S.EngineOptsT(row_groups=1))):
+            say(f"csr row groups many rows N={N} mean={mean} {name}")
+            C = torch.full((A.num_rows, N), float("nan"), device="cuda")
+            if opts is None:
+                S.spmm_csr("tiled_v3", dA, dB, C)
+            else:
+                S.spmm_tiled_v3_opts(dA, dB, opts, C)
+            torch.cuda.synchronize()
+            check_csr(C.cpu().numpy(), C64, absC)
