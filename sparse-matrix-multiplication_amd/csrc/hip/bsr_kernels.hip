@@ -16,6 +16,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <initializer_list>
 #include <type_traits>
@@ -84,30 +85,71 @@ struct BsrArgs {
     int             b_vec_ok;  // N % 8 == 0 and B 16-byte aligned
     int             block_cols;
     int             tiles_n;    // wave kernel: column tiles (grid is 1-D)
-    int             wg_total;   // wave kernel: workgroups launched
+    int             wg_total;   // wave kernel: tiles, one workgroup each
     int             xcd_order;  // wave kernel: 1 = XCD-grouped workgroup order
+    int             slices;     // record kernel: column slices where A's blocks lie in no runs
     int             num_blocks;
     int             c_vec_ok;   // C 16-byte aligned (with b_vec_ok: rows of 16-byte chunks)
 };
 
-// Workgroup -> (block-row group, column tile) for the 1-D wave-kernel grid.
+__device__ __forceinline__ int div_up(int a, int b) { return (a + b - 1) / b; }
+
+// Whether A's blocks lie in runs (banded, block-diagonal) rather than all over
+// the block-rows: of 64 entries in eight places of the list (num_blocks >= 2),
+// most are followed by the next block-column.  Every wave of a launch reads the
+// same entries and decides alike; the host cannot, A is on the device.  Only
+// one load deep: the block-rows' ends through row_ptr cost 0.4 - 0.9 us a
+// launch, scalar loads 1.5 - 2.
+struct RunSample {
+    int here, next;
+    __device__ __forceinline__ RunSample(int h, int n) : here(h), next(n) {}
+    __device__ __forceinline__ explicit RunSample(const BsrArgs& a) {
+        const int lane = threadIdx.x & 63;
+        const int from = static_cast<int>(
+            static_cast<long>(max(a.num_blocks - 9, 0)) * (lane >> 3) >> 3);
+        const int e = min(from + (lane & 7), a.num_blocks - 2);
+        here = a.col_idx[e];
+        next = a.col_idx[e + 1];
+    }
+    __device__ __forceinline__ bool in_runs() const {
+        return __popcll(__ballot(next - here == 1)) > 32;
+    }
+};
+
+// Workgroup -> (block-row group, column tile) for the 1-D wave-kernel grid; bx
+// = block_rows for a workgroup that has no tile.
 // The hardware hands workgroup L to XCD L % 8.  With xcd_order, XCD x gets
 // the contiguous logical range [x*T/8, (x+1)*T/8) (the first T % 8 XCDs one
 // more), and logical ids run column tile fastest: each XCD works on its own
 // band of block-rows with all their column tiles, so A blocks and the B rows
 // that neighbouring block-rows share are fetched into one L2 only.
-__device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int& bx, int& by) {
+// With S > 1 slices, XCDs s*8/S .. (s+1)*8/S - 1 take the s-th part of the
+// column tiles, each a band of the block-rows: its L2 holds 1/S of B.
+__device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int slices, int& bx, int& by) {
     const int L = blockIdx.x;
+    const int xcd = L & 7, idx = L >> 3;
+    if (slices > 1) {
+        const int bands = 8 / slices;
+        const int tiles = div_up(a.tiles_n, slices);
+        const int rows  = div_up(div_up(a.block_rows, 4), bands);
+        const int slice = xcd / bands;
+        const int r     = idx / tiles;
+        bx = (xcd - slice * bands) * rows + r;
+        by = slice * tiles + idx - r * tiles;
+        if (r >= rows || by >= a.tiles_n) bx = a.block_rows;
+        return;
+    }
     int l = L;
+    bool live = L < a.wg_total;
     if (a.xcd_order) {
-        const int xcd = L & 7, idx = L >> 3;
         const int per = a.wg_total >> 3, rem = a.wg_total & 7;
+        live = idx < per + (xcd < rem ? 1 : 0);
         l = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
     }
     bx = l / a.tiles_n;
     by = l - bx * a.tiles_n;
+    if (!live) bx = a.block_rows;
 }
-
 
 // ---------------------------------------------------------------------------
 // Wave kernel (pointer addressing: what the record kernel below does not take):
@@ -152,7 +194,7 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
     const int g    = lane >> 4;
     const int t    = lane & 15;
     int bx, by;
-    wave_tile_of(a, bx, by);
+    wave_tile_of(a, 1, bx, by);
     const int br   = bx * 4 + wave;
     const int n0   = by * NT;
     if (br >= a.block_rows) return;  // waves are independent: no barrier anywhere
@@ -311,7 +353,8 @@ __device__ u32x4 sbuf_load_u32x4_dev(__amdgpu_buffer_rsrc_t rsrc, int index, int
 }
 
 template <int J, int D>
-__device__ __forceinline__ void bsr_record_body(const BsrArgs& a, _Float16* __restrict__ s0,
+__device__ __forceinline__ void bsr_record_body(const BsrArgs& a, int slices,
+                                                _Float16* __restrict__ s0,
                                                 _Float16* __restrict__ s1,
                                                 _Float16* __restrict__ s2,
                                                 _Float16* __restrict__ s3) {
@@ -326,7 +369,7 @@ __device__ __forceinline__ void bsr_record_body(const BsrArgs& a, _Float16* __re
     const int g    = lane >> 4;
     const int t    = lane & 15;
     int bx, by;
-    wave_tile_of(a, bx, by);
+    wave_tile_of(a, slices, bx, by);
     const int br   = bx * 4 + wave;
     const int n0   = by * NT;
     if (br >= a.block_rows) return;  // waves are independent: no barrier anywhere
@@ -500,7 +543,8 @@ __global__ __launch_bounds__(256) void bsr_record_kernel(BsrArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 s_b1[4 * TILE];
     __shared__ __attribute__((aligned(16))) _Float16 s_b2[D == 4 ? 4 * TILE : 8];
     __shared__ __attribute__((aligned(16))) _Float16 s_b3[D == 4 ? 4 * TILE : 8];
-    bsr_record_body<J, D>(a, s_b0, s_b1, s_b2, s_b3);
+    const int slices = a.slices > 1 && !RunSample(a).in_runs() ? a.slices : 1;
+    bsr_record_body<J, D>(a, slices, s_b0, s_b1, s_b2, s_b3);
 }
 
 // ---------------------------------------------------------------------------
@@ -576,8 +620,10 @@ __device__ __forceinline__ uint64_t below(int p) {  // bits 0 .. p-1, p in [0, 6
     return (1ull << p) - 1ull;
 }
 
-template <int R, int J, int WR, int D>
-__device__ __forceinline__ void bsr_panel_body(const BsrArgs& a, _Float16* __restrict__ s0,
+// CHOOSE: returns false, with nothing done, where A's blocks lie in no runs.
+// The sample's loads go out before the panel's own and wait with them.
+template <int R, int J, int WR, int D, bool CHOOSE = false>
+__device__ __forceinline__ bool bsr_panel_body(const BsrArgs& a, _Float16* __restrict__ s0,
                                                _Float16* __restrict__ s1,
                                                _Float16* __restrict__ s2,
                                                _Float16* __restrict__ s3,
@@ -606,8 +652,11 @@ __device__ __forceinline__ void bsr_panel_body(const BsrArgs& a, _Float16* __res
     const int wr   = wave / WC;
     const int wc   = wave % WC;
     int bx, by;
-    wave_tile_of(a, bx, by);
+    wave_tile_of(a, 1, bx, by);
     const int br0 = bx * R;
+    // No tile: the whole workgroup leaves, before any barrier (or, to choose,
+    // has a panel of empty block-rows at hand).
+    if (!CHOOSE && br0 >= a.block_rows) return true;
     const int n0  = by * NT;
     auto stage = [&](int d) -> _Float16* { return d == 0 ? s0 : d == 1 ? s1 : d == 2 ? s2 : s3; };
 
@@ -616,6 +665,8 @@ __device__ __forceinline__ void bsr_panel_body(const BsrArgs& a, _Float16* __res
     const __amdgpu_buffer_rsrc_t rec_a = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<_Float16*>(a.vals), static_cast<short>(512), a.num_blocks, kBufWord3);
 
+    RunSample sample{0, 0};
+    if constexpr (CHOOSE) sample = RunSample(a);
     // Block-rows br0 .. br0+R-1 (those past the matrix are empty); their
     // lists are contiguous in col_idx from e0.
     int rp[R + 1];
@@ -643,6 +694,10 @@ __device__ __forceinline__ void bsr_panel_body(const BsrArgs& a, _Float16* __res
             lo = min(lo, a.col_idx[rp[r]]);
             hi = max(hi, a.col_idx[rp[r + 1] - 1]);
         }
+    }
+    if constexpr (CHOOSE) {
+        if (!sample.in_runs()) return false;
+        if (br0 >= a.block_rows) return true;
     }
     // Stage layout: row-major 32 x NT fp16, its 16-byte chunks XOR-swizzled
     // per row (chunk c of row r sits at position c ^ swz(r)), which spreads
@@ -949,6 +1004,7 @@ __device__ __forceinline__ void bsr_panel_body(const BsrArgs& a, _Float16* __res
             }
         }
     }
+    return true;
 }
 
 // The stages and tables are separate LDS objects passed as restrict pointers
@@ -971,6 +1027,30 @@ __global__ __launch_bounds__(256) void bsr_panel_kernel(BsrArgs a) {
                                 s_misc);
 }
 
+// One launch for wide B and 24 - 64 blocks per block-row: the shared panel
+// where A's blocks lie in runs, and the record kernel's waves (the same 4
+// block-rows x 64 columns a workgroup, in column slices) where they lie all
+// over: a panel's union then nears the sum of its lists, and its lockstep pairs
+// bound it.  The panel's stages and tables lie in the ring slots.
+__global__ __launch_bounds__(256) void bsr_wide_kernel(BsrArgs a) {
+    constexpr int R = 4, J = 4, TILE = 32 * 16 * J;
+    __shared__ __attribute__((aligned(16))) _Float16 s_b0[4 * TILE];
+    __shared__ __attribute__((aligned(16))) _Float16 s_b1[4 * TILE];
+    _Float16* const none = s_b1 + 3 * TILE;  // stages that two in flight do not have
+    uint64_t* const s_mask = reinterpret_cast<uint64_t*>(s_b1 + TILE);
+    uint32_t* const s_bits = reinterpret_cast<uint32_t*>(s_mask + 4 * R);
+    int* const s_pre  = reinterpret_cast<int*>(s_bits + kPanelMaxWords);
+    int* const s_ucol = s_pre + kPanelMaxWords;
+    int* const s_blk  = s_ucol + kPanelSlots;
+    int* const s_misc = s_blk + kPanelSlots * R;
+    static_assert(4 * R * 8 + 4 * (2 * kPanelMaxWords + kPanelSlots * (R + 1) + 8) <= 4 * TILE,
+                  "tables fit two tiles");
+    if (!bsr_panel_body<R, J, 4, 2, true>(a, s_b0, s_b1, none, none, s_bits, s_pre, s_ucol, s_blk,
+                                          s_mask, s_misc)) {
+        bsr_record_body<J, 2>(a, a.slices, s_b0, s_b1, none, none);
+    }
+}
+
 Error fail(int status, std::string msg) { return Error{status, std::move(msg)}; }
 
 Error from_hip(hipError_t e, const char* what) {
@@ -986,20 +1066,50 @@ bool records_fit(const BsrArgs& a) {
            static_cast<long long>(a.num_blocks) * 512 <= 0x7fffffffLL;
 }
 
+// Column slices for blocks that lie in no runs: as many (a power of two, at
+// most 8, splitting the tiles to within 15%) as bring an XCD's share of B to
+// about 3 MiB, which leaves its L2 room for A and C.  Each slice reads A again,
+// which costs little next to B's rows from 8 blocks per block-row on; up to 5
+// MiB B mostly stays in the L2s whole.  Below one block in 64 A is more likely a
+// band, which gains nothing and would pay for looking (32768 rows of 15 blocks, N
+// = 512: 31 -> 33 us).
+// 12288^2 at 2%: N = 512 28.2 -> 20.0 us, N = 1024 57 -> 33 us.
+int record_slices(const BsrArgs& a) {
+    const long long b_bytes = 2LL * a.K * a.N;
+    if (a.xcd_order == 0 || b_bytes <= (5LL << 20) || a.num_blocks < 8LL * a.block_rows ||
+        64LL * a.num_blocks < static_cast<long long>(a.block_rows) * a.block_cols) {
+        return 1;
+    }
+    int s = 1;
+    while (s < 8 && b_bytes > s * (3LL << 20)) s *= 2;
+    while (s > 1 && 100L * ceil_div(a.tiles_n, s) * s > 115L * a.tiles_n) s /= 2;
+    return s;
+}
+
+// Workgroups of a grid that takes either of wave_tile_of's orders.
+unsigned grid_size(const BsrArgs& a) {
+    if (a.slices == 1) return static_cast<unsigned>(a.wg_total);
+    const int rows = ceil_div(ceil_div(a.block_rows, 4), 8 / a.slices);
+    const unsigned sliced = 8u * static_cast<unsigned>(rows) * ceil_div(a.tiles_n, a.slices);
+    return std::max(sliced, static_cast<unsigned>(a.wg_total));
+}
+
 template <int J, int D>
 hipError_t run_wave(BsrArgs args, hipStream_t stream, bool pointer_addressing) {
     args.tiles_n = ceil_div(args.N, 16 * J);
     const long total = static_cast<long>(ceil_div(args.block_rows, 4)) * args.tiles_n;
     if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
     args.wg_total = static_cast<int>(total);
-    dim3 grid(args.wg_total);
+    args.slices = record_slices(args);
+    const unsigned tiles = grid_size(args);
     if (!pointer_addressing && records_fit(args)) {
-        hipLaunchKernelGGL((bsr_record_kernel<J, D == 1 ? 2 : D>), grid, dim3(256), 0, stream,
-                           args);
+        hipLaunchKernelGGL((bsr_record_kernel<J, D == 1 ? 2 : D>), dim3(tiles), dim3(256), 0,
+                           stream, args);
         return hipGetLastError();
     }
     if (static_cast<long long>(args.K) * args.N >= 8) {
-        hipLaunchKernelGGL((bsr_wave_kernel<J, D, true>), grid, dim3(256), 0, stream, args);
+        hipLaunchKernelGGL((bsr_wave_kernel<J, D, true>), dim3(args.wg_total), dim3(256), 0,
+                           stream, args);
     } else {  // B is smaller than one chunk
         args.tiles_n  = 1;
         args.wg_total = ceil_div(args.block_rows, 4);
@@ -1025,6 +1135,16 @@ hipError_t run_panel(BsrArgs args, hipStream_t stream) {
     args.wg_total = static_cast<int>(total);
     hipLaunchKernelGGL((bsr_panel_kernel<R, J, WR, D>), dim3(args.wg_total), dim3(256), 0, stream,
                        args);
+    return hipGetLastError();
+}
+
+hipError_t run_wide(BsrArgs args, hipStream_t stream) {
+    args.tiles_n = ceil_div(args.N, 64);
+    const long total = static_cast<long>(ceil_div(args.block_rows, 4)) * args.tiles_n;
+    if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
+    args.wg_total = static_cast<int>(total);
+    args.slices = record_slices(args);
+    hipLaunchKernelGGL(bsr_wide_kernel, dim3(grid_size(args)), dim3(256), 0, stream, args);
     return hipGetLastError();
 }
 
@@ -1085,6 +1205,7 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
                  0,
                  0,
                  0,
+                 1,
                  A.num_blocks,
                  reinterpret_cast<uintptr_t>(C) % 16 == 0 ? 1 : 0};
     const BsrOpts o = opts ? *opts : BsrOpts{};
@@ -1117,14 +1238,27 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
     const bool rec = o.addressing != 1 && records_fit(args);
     const double bpr = A.block_rows > 0 ? static_cast<double>(A.num_blocks) / A.block_rows : 0.0;
     // Shared-panel kernel (R = 4, 64 columns, 2 stages): automatic on wide B
-    // with long block-rows of structured inputs, the cells where it measured
-    // faster than the wave kernel (N >= 256, 24 - 64 blocks per block-row:
-    // 1.03 - 1.31x over 36 block-diagonal and banded inputs); explicit
-    // row_group 4 / 8 forces it.
+    // with long block-rows, where it measured faster than the wave kernel on
+    // structured inputs (N >= 256, 24 - 64 blocks per block-row: 1.03 - 1.31x
+    // over 36 block-diagonal and banded inputs); explicit row_group 4 / 8
+    // forces it.  From one block in 24 on A may as well have no structure, and
+    // then the panel takes 1.6 - 3.4 times the waves' time, so from N = 320 each
+    // launch looks (bsr_wide_kernel; against the panel: blocks at 12.5% of
+    // 8192^2, N = 512 62 -> 40 us and N = 1024 119 -> 76; 3000 x 6997 at 10%, N =
+    // 512 43 -> 14; bands and diagonal blocks within 3%), and below the waves are
+    // level on structured inputs too (12.5%, N = 256: 59 -> 19.6 us; bands 8.8 ->
+    // 8.6 and 13.4 -> 13.8, diagonal blocks of 1024 12.1 -> 8.8).  Sparser A keeps the
+    // panel: bands of 16384 rows, N = 256 take 15.0 us there, 16.8 with waves.
     const bool panel_auto = rec && N >= 256 && A.block_cols <= kPanelMaxWords * 32 &&
                             bpr >= 24.0 && bpr <= 64.0;
+    const bool dense = 24.0 * bpr >= A.block_cols;
+    const bool defaults = !o.per_wave && o.row_group == 0 && o.tiles == 0 && o.depth == 0;
+    if (panel_auto && dense && defaults && N >= 320) {
+        return from_hip(run_wide(args, stream), "spmm_wmma launch");
+    }
     const bool panel = !o.per_wave && rec &&
-                       (o.row_group == 4 || o.row_group == 8 || (o.row_group == 0 && panel_auto));
+                       (o.row_group == 4 || o.row_group == 8 ||
+                        (o.row_group == 0 && panel_auto && !(dense && defaults)));
     if (panel) {
         const int R = o.row_group == 8 ? 8 : 4;
         const int j = o.tiles == 8 ? 8 : 4;

@@ -432,3 +432,40 @@ def test_wmma_any_width_and_alignment(S, O, torch, N, shift):
             check_csr(dC.cpu().numpy(), C64, absC, tol=1e-5)
             assert torch.isnan(cbuf[:4 + shift]).all()
             assert torch.isnan(cbuf[4 + shift + M * N:]).all()
+
+
+@pytest.mark.parametrize("pattern", ["strewn", "runs", "both"])
+@pytest.mark.parametrize("M,K,N", [(1007, 1600, 320), (530, 1293, 648), (2100, 8200, 512),
+                                   (100, 5300, 1024)])
+def test_wmma_wide_b(S, O, torch, pattern, M, K, N):
+    # Wide B and 24 - 64 blocks per block-row: blocks in runs take the shared
+    # panel, others the waves, over column slices where B is over 5 MiB; row
+    # groups and column tiles that the XCDs' shares do not divide.
+    rng = np.random.default_rng(M + N)
+    br, bc = -(-M // 16), -(-K // 16)
+    row_ptr, cols = [0], []
+    for r in range(br):
+        count = min(bc, 26 + r % 37)
+        if pattern == "runs" or (pattern == "both" and r % 2):
+            c = np.arange(count) + (r * 3) % (bc - count + 1)
+        else:
+            c = np.sort(rng.choice(bc, count, replace=False))
+        cols.append(c)
+        row_ptr.append(row_ptr[-1] + count)
+    cols = np.concatenate(cols).astype(np.int32)
+    vals = rng.uniform(-1, 1, (cols.size, 16, 16)).astype(np.float16)
+    last_row = np.repeat(np.arange(br), np.diff(row_ptr)) * 16
+    vals[(last_row[:, None] + np.arange(16) >= M)] = 0
+    vals.transpose(0, 2, 1)[cols[:, None] * 16 + np.arange(16) >= K] = 0
+    hb = S.HostBSR(M, K, br, bc, int(np.count_nonzero(vals)), np.array(row_ptr, np.int32), cols,
+                   vals.reshape(-1).view(np.uint16))
+    B16 = rng.uniform(-1, 1, (K, N)).astype(np.float16)
+    C32 = O.bsr_spmm_f32(M, K, hb.row_ptr, hb.col_idx, hb.values, B16.view(np.uint16))
+    dense = np.zeros((br, bc, 16, 16))
+    dense[np.repeat(np.arange(br), np.diff(row_ptr)), cols] = vals
+    dense = dense.transpose(0, 2, 1, 3).reshape(br * 16, bc * 16)[:M, :K]
+    C64, absC = dense @ B16.astype(np.float64), np.abs(dense) @ np.abs(B16.astype(np.float64))
+    say(f"wmma wide B {pattern} M={M} K={K} N={N} blocks={cols.size}")
+    C = _run_wmma(S, torch, hb, B16.view(np.uint16))
+    check_bsr(C, C32, absC)
+    check_csr(C, C64, absC, tol=1e-5)
