@@ -116,8 +116,10 @@ typedef struct spmm_engine_opts_t {
 
 /* BSR matrix-core kernel tuning (0 = automatic).  No counterpart in the
  * reference: exposes the kernels' variants for measurement sweeps.  Default:
- * the shared-panel kernel on wide B with long structured block-rows (N >= 256,
- * 24 - 64 blocks per block-row on average, K <= 131072), else the wave kernel. */
+ * the shared-panel kernel on wide B with long block-rows (N >= 256, 24 - 64
+ * blocks per block-row on average, K <= 131072), else the wave kernel.  From one
+ * block in 24 on the wave kernel for N < 320, and for wider B one launch that
+ * takes the panel where A's blocks lie in runs and waves where they do not. */
 typedef struct spmm_bsr_opts_t {
     int row_group;  /* 0: automatic; 1: wave kernel (one wave per block-row);
                        4, 8: shared-panel kernel with that many block-rows per
