@@ -581,8 +581,8 @@ __global__ __launch_bounds__(256) void bsr_record_kernel(BsrArgs a) {
 // -- so the panel saves L1 accesses (0.66 M vs 1.44 M of 64 bytes) but pays
 // barriers, lockstep phases and LDS read bandwidth.  It is faster only on
 // wide B with long block-rows (N >= 256 and 24 - 64 blocks per block-row:
-// 1.03 - 1.31x, e.g. block-diagonal 512 at N = 512 12.6 -> 10.8 us), which is
-// where the launcher picks it; c3 and c4 stay on the wave kernel.
+// 1.03 - 1.31x, e.g. block-diagonal 512 at N = 512 12.6 -> 10.8 us), and
+// the launcher picks it there for A in runs; c3 and c4 stay on the wave kernel.
 // ---------------------------------------------------------------------------
 constexpr int kPanelMaxWords = 256;  // union bitmap: up to 8192 block-columns (K <= 131072)
 constexpr int kPanelSlots    = 126;  // union slots per pass (two registers per lane, lane 127 free)
