@@ -85,7 +85,14 @@ __device__ __forceinline__ typename Vec<VEC>::T vzero() {
 // gathers its B segment with a bounds-checked buffer load (one record per B
 // row, so the row index is the load's index operand and needs no address
 // arithmetic).  Each register of the U rows in flight is refilled as soon as it
-// is used, and the entries are read from LDS one step ahead.  At a row's end:
+// is used, and the entries are read from LDS one step ahead.  Every fourth entry
+// of a range goes to the same of four partial sums (kChains), added at a row's
+// end: the rounding error grows with the longest chain, and one chain per range
+// is up to twice as far from 64 bits as the interleaved groups of
+// csr_rowblock_wide (merge-path parts of 30000^2, 120 per row, N = 32: 1.8e-7 of the
+// norm, with four 1.0e-7; 65536^2, 32 per row, N = 256 8.2e-8 and 6.5e-8).  They cost
+// a row end 24 instructions (16384^2, 8 per row, N = 128 9.4 -> 10.4 us; 65536^2, 32
+// per row, N = 256 210 -> 208).  At a row's end:
 //   - a row that lies wholly inside the group's range is stored to C;
 //   - the first row of a range that started in an earlier group goes to an LDS
 //     slot of the group;
@@ -165,6 +172,7 @@ constexpr int kRpCap = 1024;  // row pointers staged per window
 constexpr int kWCap  = 256;   // (col, value) entries a wave stages at a time
 constexpr int kMinWindow = 16;  // entries of a group's window: two steps
 constexpr int kMaxGroups = kWCap / kMinWindow;  // lane groups of a wave
+constexpr int kChains = 4;  // interleaved sums of a row in csr_rowblock
 
 // Third dword of a gfx9 buffer resource: 32-bit data format, no swizzle.
 constexpr int kBufWord3 = 0x00020000;
@@ -320,9 +328,10 @@ __device__ __forceinline__ float entry_value(Entry e) {
 }
 
 template <int VEC, int WAVES, int U, bool SBUF, bool HALVES>
-__global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
+__global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(RowblockArgs a) {
     using VT = typename Vec<VEC>::T;
     static_assert(kWCap % kWave == 0 && kMinWindow % U == 0, "whole steps per window");
+    static_assert(U % kChains == 0, "an entry's chain is fixed by its place in the step");
 
     __shared__ int  s_rp[kRpCap + 2];
     __shared__ VT   s_part[WAVES * kWave];   // by group and lane: the group's head piece
@@ -334,13 +343,22 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     const int wave  = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lpg   = a.group_lanes;
     const int G     = a.groups;
-    // Lanes past the last group shadow its last lane and never store.
-    const int grp   = min(lane * a.lanes_inv >> 16, G - 1);
-    const int glane = min(lane - grp * lpg, lpg - 1);
-    const bool live = lane < G * lpg;
-    const int gi    = wave * G + grp;  // group of the workgroup
     const int NG    = WAVES * G;
-    VT* const my_part = s_part + gi * lpg + glane;
+    // A lane's place.  Lanes past the last group shadow its last lane and never
+    // store.  Worked out anew where it is needed: held over the entry loop it
+    // would take registers from the rows in flight.
+    struct Place {
+        int  grp, glane;
+        int  gi;  // group of the workgroup
+        bool live;
+    };
+    auto place = [&] {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        const int g  = min(l * a.lanes_inv >> 16, G - 1);
+        const int gl = min(l - g * lpg, lpg - 1);
+        return Place{g, gl, wave * G + g, l < G * lpg};
+    };
     const int N     = a.N;
     const int cap   = 1 << a.window_log;  // entries a group stages at a time
     const int cols  = lpg * VEC;          // columns per pass
@@ -394,8 +412,12 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
     // A group's window and the 2U empty entries that the last steps' loads may
     // read; an odd stride puts the groups' windows on different banks.
     const int kv_len  = cap + 2 * U + 1;
-    const int kv_mine = grp * kv_len;
-    for (int i = glane; i <= 2 * U; i += lpg) kv[kv_mine + cap + i] = entry(SBUF ? -1 : 0, 0.0f);
+    {
+        const Place me = place();
+        for (int i = me.glane; i <= 2 * U; i += lpg) {
+            kv[me.grp * kv_len + cap + i] = entry(SBUF ? -1 : 0, 0.0f);
+        }
+    }
 
     for (int w0 = r_begin; w0 < r_end; w0 += kRpCap) {
         const int nr = min(r_end - w0, kRpCap);
@@ -431,6 +453,7 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
             (static_cast<int>(__umulhi(total, a.groups_inv)) / WAVES + U) / U * U;
         const unsigned rest = total;
         const unsigned from = min(rest, static_cast<unsigned>(wave * G) * share);  // the wave's first
+        const int gi   = place().gi;
         const int pa   = nz0 + static_cast<int>(min(rest, static_cast<unsigned>(gi) * share));
         const int pb   = nz0 + static_cast<int>(min(rest, static_cast<unsigned>(gi + 1) * share));
         const int wlen = static_cast<int>(min<unsigned>(share, rest - from));  // its longest range
@@ -489,13 +512,38 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
         if (wlen > 0 && one_window) stage(0);
 
         for (int c0 = cbeg; c0 < cend; c0 += cols) {
-            const int  col    = lane_col<VEC>(c0 + glane * VEC, cend);
-            const bool writer = live && c0 + glane * VEC < cend;
-            const float* bcol = m.B + col;
-            if (live && glane == 0) s_first[gi] = -1;
+            int  colb;    // byte offset of the lane's columns
+            bool writer;  // whether the lane stores them
+            {
+                const Place me = place();
+                colb   = lane_col<VEC>(c0 + me.glane * VEC, cend) * 4;
+                writer = me.live && c0 + me.glane * VEC < cend;
+                if (me.live && me.glane == 0) s_first[me.gi] = -1;
+            }
+            const float* bcol = reinterpret_cast<const float*>(reinterpret_cast<const char*>(m.B) + colb);
+            // Puts v aside as the group's piece of local row r.
+            auto put_piece = [&](int r, VT v) {
+                const Place me = place();
+                if (me.live) s_part[me.gi * lpg + me.glane] = v;
+                if (me.live && me.glane == 0) s_first[me.gi] = r;
+            };
+            auto store_row = [&](float* base, unsigned r, VT v) {
+                unsigned cb = colb;
+                asm volatile("" : "+v"(cb));  // keeps base + cb out of the entry loop's registers
+                if (writer) {
+                    store_vec<VEC>(reinterpret_cast<float*>(
+                        reinterpret_cast<char*>(base) + (static_cast<size_t>(r) * (4u * N) + cb)), v);
+                }
+            };
 
             int owner_row = -1;  // local row this group finishes after the barrier
-            VT acc = vzero<VEC>();
+            VT acc[kChains];
+            const auto clear = [&] {
+#pragma unroll
+                for (int i = 0; i < kChains; ++i) acc[i] = vzero<VEC>();
+            };
+            const auto sum = [&] { return (acc[0] + acc[1]) + (acc[2] + acc[3]); };
+            clear();
             if (wlen > 0) {
                 int  row  = first;
                 bool head = s_rp[row] < pa;  // row began in an earlier group
@@ -510,14 +558,14 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                 int next_end = s_rp[row + 2 <= nr ? row + 2 : nr];
 
                 auto flush = [&](int at) {
+                    const VT done = sum();
                     if (head) {
-                        if (live) *my_part = acc;
-                        if (live && glane == 0) s_first[gi] = row;
+                        put_piece(row, done);
                         head = false;
-                    } else if (writer) {
-                        store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, acc);
+                    } else {
+                        store_row(m.C, w0 + row, done);
                     }
-                    acc = vzero<VEC>();
+                    clear();
                     ++row;
                     int e = next_end;
                     while (e <= at + pa && row < nr - 1) {  // empty rows
@@ -538,11 +586,11 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                     VT    bv[U];
                     float vv[U];
                     Entry next[U];
-                    int at_kv = kv_mine;
+                    int at_kv = place().grp * kv_len;
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         vv[u] = entry_value(kv[at_kv + u]);
-                        bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(kv[at_kv + u]), col * 4, N);
+                        bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(kv[at_kv + u]), colb, N);
                     }
 #pragma unroll
                     for (int u = 0; u < U; ++u) next[u] = kv[at_kv + U + u];
@@ -555,11 +603,12 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                             if (__builtin_expect(ends, 0)) {
                                 if (at0 + u == row_len) flush(at0 + u);
                             }
-                            if (SBUF || at0 + u < pb - pa) acc = vv[u] * bv[u] + acc;
+                            VT& a_u = acc[u % kChains];
+                            if (SBUF || at0 + u < pb - pa) a_u = vv[u] * bv[u] + a_u;
                             if constexpr (decltype(refill)::value) {
                                 __builtin_amdgcn_sched_barrier(0);  // into the registers just used
                                 vv[u] = entry_value(next[u]);
-                                bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(next[u]), col * 4, N);
+                                bv[u] = load_b<VEC, SBUF>(rsrc, bcol, entry_row(next[u]), colb, N);
                                 next[u] = kv[at_kv + 2 * U + u];
                                 __builtin_amdgcn_sched_barrier(0);  // a step ahead of its use
                             }
@@ -574,34 +623,35 @@ __global__ __launch_bounds__(WAVES * 64) void csr_rowblock(RowblockArgs a) {
                     step(win + q, std::false_type());
                 }
                 // The row being accumulated when the range ends.
+                acc[0] = sum();
                 if (pa < pb) {
                     if (head) {
-                        if (live) *my_part = acc;
-                        if (live && glane == 0) s_first[gi] = row;
+                        put_piece(row, acc[0]);
                     } else if (s_rp[row + 1] <= pb) {
-                        if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + row) * N + col, acc);
+                        store_row(m.C, w0 + row, acc[0]);
                     } else {
                         owner_row = row;
                     }
                 }
             }
             __syncthreads();
+            const Place me = place();
             if (owner_row >= 0) {
-                for (int w = gi + 1; w < NG; ++w) {
+                for (int w = me.gi + 1; w < NG; ++w) {
                     if (s_first[w] != owner_row) break;
-                    acc += s_part[w * lpg + glane];
+                    acc[0] += s_part[w * lpg + me.glane];
                 }
-                if (writer) store_vec<VEC>(m.C + static_cast<size_t>(w0 + owner_row) * N + col, acc);
+                store_row(m.C, w0 + owner_row, acc[0]);
             }
-            if (wg_head >= 0 && w0 == r_begin && gi == 0) {
+            if (wg_head >= 0 && w0 == r_begin && me.gi == 0) {
                 // The part's first row began in an earlier part: the groups that
                 // hold pieces of it (local row 0, leading groups) go to the carry.
-                VT sum = vzero<VEC>();
+                VT piece = vzero<VEC>();
                 for (int w = 0; w < NG; ++w) {
                     if (s_first[w] != 0) break;
-                    sum += s_part[w * lpg + glane];
+                    piece += s_part[w * lpg + me.glane];
                 }
-                if (writer) store_vec<VEC>(m.carry + static_cast<size_t>(rb) * N + col, sum);
+                store_row(m.carry, rb, piece);
             }
             __syncthreads();  // s_part / s_first are rewritten by the next column pass
         }

@@ -592,3 +592,40 @@ def test_row_groups_many_rows(S, O, torch, N):
                 S.spmm_tiled_v3_opts(dA, dB, opts, C)
             torch.cuda.synchronize()
             check_csr(C.cpu().numpy(), C64, absC)
+
+
+@pytest.mark.parametrize("N", [24, 64, 100])
+def test_engine_rounding(S, O, torch, N):
+    # A row is summed in four interleaved chains (of a lane group's range, whose
+    # pieces are added in order), so its rounding error is at most that of four
+    # fp32 chains over whole rows, here computed on the CPU, and far below one
+    # chain's.  1.1: ranges of a few entries end chains early, which moves the
+    # error by a few percent either way.
+    M, K, per = 1500, 2000, 160
+    rng = np.random.default_rng(5)
+    col = np.sort(rng.random((M, K)).argpartition(per, 1)[:, :per], 1).astype(np.int32)
+    val = rng.uniform(-1, 1, (M, per)).astype(np.float32)
+    A = S.HostCSR(M, K, np.arange(M + 1, dtype=np.int32) * per, col.ravel(), val.ravel())
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    C64, absC = O.csr_spmm_f64(A.row_ptr, A.col_idx, A.values, B)
+    chains = np.zeros((4, M, N), np.float32)
+    for e in range(per):  # a product of fp32 is exact in fp64: one rounding, as a fused step
+        chains[e % 4] = (val[:, e, None].astype(np.float64) * B[col[:, e]] + chains[e % 4]).astype(np.float32)
+    four = (chains[0] + chains[1]) + (chains[2] + chains[3])
+    bound = 1.1 * np.linalg.norm(four - C64) / np.linalg.norm(C64)
+    dA, dB = S.DeviceCSR(A), torch.from_numpy(B).cuda()
+    rows = torch.from_numpy(S.nnz_split_rows(A, 16)).cuda()
+    E = S.EngineOptsT
+    runs = {"engine": lambda: S.spmm_tiled_v3_opts(dA, dB, E(vec=4)),
+            "vec2": lambda: S.spmm_tiled_v3_opts(dA, dB, E(vec=2, groups=1)),
+            "unroll8": lambda: S.spmm_tiled_v3_opts(dA, dB, E(vec=4, unroll=8)),
+            "pointers": lambda: S.spmm_tiled_v3_opts(dA, dB, E(global_loads=1)),
+            "long ranges": lambda: S.spmm_tiled_v3_opts(dA, dB, E(vec=4, waves=2, rows_per_block=512)),
+            "split": lambda: S.spmm_tiled_v3_split(dA, rows, dB)}
+    for name, run in runs.items():
+        say(f"csr engine rounding {name} N={N}")
+        C = run().cpu().numpy()
+        rel = check_csr(C, C64, absC)
+        # One or two groups on merge-path parts take alternate entries instead:
+        # two chains, or one per row at N over 128.
+        assert rel <= bound * (1.5 if name == "split" and N == 100 else 1.0), (name, rel, bound)
