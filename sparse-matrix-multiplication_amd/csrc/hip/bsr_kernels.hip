@@ -87,6 +87,7 @@ struct BsrArgs {
     int             tiles_n;    // wave kernel: column tiles (grid is 1-D)
     int             wg_total;   // wave kernel: tiles, one workgroup each
     int             xcd_order;  // wave kernel: 1 = XCD-grouped workgroup order
+    int             sample_step;  // between the eight places of RunSample
     int             slices;     // record kernel: column slices where A's blocks lie in no runs
     int             num_blocks;
     int             c_vec_ok;   // C 16-byte aligned (with b_vec_ok: rows of 16-byte chunks)
@@ -95,24 +96,20 @@ struct BsrArgs {
 __device__ __forceinline__ int div_up(int a, int b) { return (a + b - 1) / b; }
 
 // Whether A's blocks lie in runs (banded, block-diagonal) rather than all over
-// the block-rows: of 64 entries in eight places of the list (num_blocks >= 2),
-// most are followed by the next block-column.  Every wave of a launch reads the
-// same entries and decides alike; the host cannot, A is on the device.  Only
-// one load deep: the block-rows' ends through row_ptr cost 0.4 - 0.9 us a
-// launch, scalar loads 1.5 - 2.
+// the block-rows: of eight entries in each of eight places of the list
+// (num_blocks >= 8), most are followed by the next block-column.  Every wave of
+// a launch reads the same entries and decides alike; the host cannot, A is on
+// the device.  Only one load deep: the block-rows' ends through row_ptr cost 0.4
+// - 0.9 us a launch, scalar loads 1.5 - 2.
 struct RunSample {
-    int here, next;
-    __device__ __forceinline__ RunSample(int h, int n) : here(h), next(n) {}
-    __device__ __forceinline__ explicit RunSample(const BsrArgs& a) {
+    int here = 0;
+    __device__ __forceinline__ void load(const BsrArgs& a) {
         const int lane = threadIdx.x & 63;
-        const int from = static_cast<int>(
-            static_cast<long>(max(a.num_blocks - 9, 0)) * (lane >> 3) >> 3);
-        const int e = min(from + (lane & 7), a.num_blocks - 2);
-        here = a.col_idx[e];
-        next = a.col_idx[e + 1];
+        here = a.col_idx[(lane >> 3) * a.sample_step + (lane & 7)];
     }
     __device__ __forceinline__ bool in_runs() const {
-        return __popcll(__ballot(next - here == 1)) > 32;
+        const int next = __builtin_amdgcn_update_dpp(here, here, 0x101, 0xF, 0xF, false);  // row_shl:1
+        return __popcll(__ballot(next - here == 1 && (threadIdx.x & 7) != 7)) > 28;  // of 56
     }
 };
 
@@ -543,7 +540,12 @@ __global__ __launch_bounds__(256) void bsr_record_kernel(BsrArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 s_b1[4 * TILE];
     __shared__ __attribute__((aligned(16))) _Float16 s_b2[D == 4 ? 4 * TILE : 8];
     __shared__ __attribute__((aligned(16))) _Float16 s_b3[D == 4 ? 4 * TILE : 8];
-    const int slices = a.slices > 1 && !RunSample(a).in_runs() ? a.slices : 1;
+    int slices = a.slices;
+    if (slices > 1) {
+        RunSample sample;
+        sample.load(a);
+        if (sample.in_runs()) slices = 1;
+    }
     bsr_record_body<J, D>(a, slices, s_b0, s_b1, s_b2, s_b3);
 }
 
@@ -665,8 +667,8 @@ __device__ __forceinline__ bool bsr_panel_body(const BsrArgs& a, _Float16* __res
     const __amdgpu_buffer_rsrc_t rec_a = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<_Float16*>(a.vals), static_cast<short>(512), a.num_blocks, kBufWord3);
 
-    RunSample sample{0, 0};
-    if constexpr (CHOOSE) sample = RunSample(a);
+    RunSample sample;
+    if constexpr (CHOOSE) sample.load(a);
     // Block-rows br0 .. br0+R-1 (those past the matrix are empty); their
     // lists are contiguous in col_idx from e0.
     int rp[R + 1];
@@ -1027,27 +1029,176 @@ __global__ __launch_bounds__(256) void bsr_panel_kernel(BsrArgs a) {
                                 s_misc);
 }
 
+// The waves of bsr_wide_kernel: the record kernel's work of four 16-column tiles,
+// with single blocks (not pairs) following each other through three slots.  A
+// block's loads go out two blocks ahead, about as far ahead as of pairs in two
+// slots, in 6 KiB a wave instead of eight: five of these workgroups fit a CU, as
+// of the panel kernel's, where 32 KiB would hold four (LDS is given out in 1280
+// bytes).
+__device__ __forceinline__ void bsr_wide_waves(const BsrArgs& a, int slices,
+                                               _Float16* __restrict__ s0,
+                                               _Float16* __restrict__ s1,
+                                               _Float16* __restrict__ s2) {
+    constexpr int BLOCK = 16 * 64;  // fp16 of a slot: 16 B rows x 64 columns
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g    = lane >> 4;
+    const int t    = lane & 15;
+    int bx, by;
+    wave_tile_of(a, slices, bx, by);
+    const int br = bx * 4 + wave;
+    const int n0 = by * 64;
+    if (br >= a.block_rows) return;  // waves are independent: no barrier anywhere
+    auto slot = [&](int i) -> _Float16* { return (i == 0 ? s0 : i == 1 ? s1 : s2) + wave * BLOCK; };
+
+    const __amdgpu_buffer_rsrc_t rec_b = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16*>(a.B), static_cast<short>(a.N * 2), a.K, kBufWord3);
+    const __amdgpu_buffer_rsrc_t rec_a = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16*>(a.vals), static_cast<short>(512), a.num_blocks, kBufWord3);
+
+    // Load c of a block fills rows 8c .. 8c+7 of the slot, lane l row l / 8 of
+    // them and 16-byte position l % 8, which holds chunk l % 8 ^ swz (rows 8
+    // apart swizzle alike): the eight rows that half a wave reads at once then
+    // lie on all banks.  Columns past N read a valid chunk and are not stored.
+    auto swz = [](int r) { return 2 * ((r >> 1) & 3); };
+    const int srow  = lane >> 3;
+    const int n     = n0 + ((lane & 7) ^ swz(srow)) * 8;
+    const int nbyte = (n < a.N ? n : 0) * 2;
+    // B operand: rows 4g .. 4g+3, column t of each tile; A operand: row t,
+    // columns 4g .. 4g+3.
+    const int brow = 4 * g + (t >> 2);
+    const int h    = swz(brow) >> 1;
+    const int in   = brow * 64 + ((t & 3) >> 1) * 8 + (t & 1) * 4;  // fp16 units
+    const int a_off = t * 32 + 8 * g;
+
+    const int bs = a.row_ptr[br];
+    const int be = a.row_ptr[br + 1];
+    f32x4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4(0.0f);
+    u32x2 af[3];
+
+    for (int c0 = bs; c0 < be; c0 += 64) {  // 64 blocks per column-index chunk
+        const int cnt = min(64, be - c0);
+        const int ci  = lane < cnt ? a.col_idx[c0 + lane] : 0;
+        auto load = [&](int q, int k) {  // block c0 + q into slot k
+            const int bc  = __builtin_amdgcn_readlane(ci, q);
+            _Float16* dst = slot(k);
+            sbuf_load_lds(rec_b, (spmm_lds_ptr)dst, 16, bc * 16 + srow, nbyte, 0, 0, 0);
+            sbuf_load_lds(rec_b, (spmm_lds_ptr)(dst + 512), 16, bc * 16 + 8 + srow, nbyte, 0, 0, 0);
+            af[k] = sbuf_load_u32x2(rec_a, c0 + q, a_off, 0, 0);
+        };
+        auto multiply = [&](int k) {
+            const f16x4 afv = __builtin_bit_cast(f16x4, af[k]);
+            const _Float16* st = slot(k);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const s16x4 b = lds_read_tr16(st + in + (j ^ h) * 16);
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(afv, __builtin_bit_cast(f16x4, b),
+                                                               acc[j], 0, 0, 0);
+            }
+        };
+        // The loads of the two blocks after q, three each, may still be under
+        // way when q is multiplied (loads retire in issue order).
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (k < cnt) load(k, k);
+        }
+        int q0 = 0;
+        for (; q0 + 5 < cnt; q0 += 3) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                wait_vmcnt<6>();
+                multiply(k);
+                load(q0 + k + 3, k);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {  // the last 1 .. 5 blocks
+            if (q0 + k < cnt) {
+                if (q0 + k + 2 < cnt) wait_vmcnt<6>();
+                else if (q0 + k + 1 < cnt) wait_vmcnt<3>();
+                else wait_vmcnt<0>();
+                multiply(k % 3);
+                if (q0 + k + 3 < cnt) load(q0 + k + 3, k % 3);
+            }
+        }
+    }
+
+    // D layout: lane holds rows 4*g + i, column t of each 16-column tile.
+    const int rows_here = min(16, a.M - br * 16);
+    if (a.c_vec_ok) {
+        // As in the record kernel, two tiles through a slot at a time: 16 rows of
+        // 32 floats, stored as 128-byte row pieces.
+        const __amdgpu_buffer_rsrc_t c_rows = __builtin_amdgcn_make_buffer_rsrc(
+            a.C + static_cast<size_t>(br) * 16 * a.N, static_cast<short>(0),
+            rows_here * a.N * 4, kBufWord3);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float* ct = reinterpret_cast<float*>(slot(h));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ct[(4 * g + i) * 32 + 16 * j + t] = acc[2 * h + j][i];
+            }
+            const int col = n0 + 32 * h + (lane & 7) * 4;  // N % 8 == 0: all in or all out
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int r   = s * 8 + (lane >> 3);
+                const f32x4 v = *reinterpret_cast<const f32x4*>(ct + r * 32 + (lane & 7) * 4);
+                if (r < rows_here && col < a.N) {
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), c_rows,
+                                                           (r * a.N + col) * 4, 0, kStoreDevice);
+                }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int col = n0 + 16 * j + t;
+        if (col >= a.N) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = br * 16 + 4 * g + i;
+            if (row < a.M) store_c(a.C + static_cast<size_t>(row) * a.N + col, acc[j][i]);
+        }
+    }
+}
+
 // One launch for wide B and 24 - 64 blocks per block-row: the shared panel
-// where A's blocks lie in runs, and the record kernel's waves (the same 4
-// block-rows x 64 columns a workgroup, in column slices) where they lie all
-// over: a panel's union then nears the sum of its lists, and its lockstep pairs
-// bound it.  The panel's stages and tables lie in the ring slots.
+// where A's blocks lie in runs, and waves (the same 4 block-rows x 64 columns a
+// workgroup, in column slices) where they lie all over: a panel's union then
+// nears the sum of its lists, and its lockstep pairs bound it.  The panel's
+// stages lie in the waves' slots.  PAIRS: the waves are the record kernel's, whose
+// 32 KiB of slots leave a CU four workgroups; else bsr_wide_waves and five.
+constexpr int kWideTables = 4 * (2 * kPanelMaxWords + kPanelSlots * 5 + 8) + 8 * 16;  // bytes
+constexpr bool cu_holds(int workgroups, int lds_bytes) {  // LDS: 160 KiB, given out in 1280 bytes
+    return workgroups * ((lds_bytes + 1279) / 1280) <= 128;
+}
+static_assert(cu_holds(4, 4 * 2 * 4096 + kWideTables + 16) && cu_holds(5, 4 * 3 * 2048 + kWideTables),
+              "resident workgroups of the two forms of bsr_wide_kernel");
+
+template <bool PAIRS>
 __global__ __launch_bounds__(256) void bsr_wide_kernel(BsrArgs a) {
-    constexpr int R = 4, J = 4, TILE = 32 * 16 * J;
-    __shared__ __attribute__((aligned(16))) _Float16 s_b0[4 * TILE];
-    __shared__ __attribute__((aligned(16))) _Float16 s_b1[4 * TILE];
-    _Float16* const none = s_b1 + 3 * TILE;  // stages that two in flight do not have
-    uint64_t* const s_mask = reinterpret_cast<uint64_t*>(s_b1 + TILE);
-    uint32_t* const s_bits = reinterpret_cast<uint32_t*>(s_mask + 4 * R);
-    int* const s_pre  = reinterpret_cast<int*>(s_bits + kPanelMaxWords);
-    int* const s_ucol = s_pre + kPanelMaxWords;
-    int* const s_blk  = s_ucol + kPanelSlots;
-    int* const s_misc = s_blk + kPanelSlots * R;
-    static_assert(4 * R * 8 + 4 * (2 * kPanelMaxWords + kPanelSlots * (R + 1) + 8) <= 4 * TILE,
-                  "tables fit two tiles");
-    if (!bsr_panel_body<R, J, 4, 2, true>(a, s_b0, s_b1, none, none, s_bits, s_pre, s_ucol, s_blk,
+    constexpr int R = 4, J = 4, STAGE = 32 * 16 * J, SLOT = PAIRS ? 4 * STAGE : 2 * STAGE;
+    __shared__ __attribute__((aligned(16))) _Float16 s_b0[SLOT];
+    __shared__ __attribute__((aligned(16))) _Float16 s_b1[SLOT];
+    __shared__ __attribute__((aligned(16))) _Float16 s_b2[PAIRS ? 8 : SLOT];
+    __shared__ uint32_t s_bits[kPanelMaxWords];
+    __shared__ int s_pre[kPanelMaxWords];
+    __shared__ int s_ucol[kPanelSlots];
+    __shared__ int s_blk[kPanelSlots * R];
+    __shared__ uint64_t s_mask[4 * R];
+    __shared__ int s_misc[8];
+    // two stages: the other two are never touched
+    if (!bsr_panel_body<R, J, 4, 2, true>(a, s_b0, s_b1, s_b2, s_b2, s_bits, s_pre, s_ucol, s_blk,
                                           s_mask, s_misc)) {
-        bsr_record_body<J, 2>(a, a.slices, s_b0, s_b1, none, none);
+        if constexpr (PAIRS) {
+            bsr_record_body<J, 2>(a, a.slices, s_b0, s_b1, s_b2, s_b2);
+        } else {
+            bsr_wide_waves(a, a.slices, s_b0, s_b1, s_b2);
+        }
     }
 }
 
@@ -1138,13 +1289,25 @@ hipError_t run_panel(BsrArgs args, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Workgroups up to which the wide kernel's waves take pairs: four per CU.  The
+// panel loses nothing to 32 KiB of slots then and the waves gain (MI355X, blocks
+// at 12.5% of 8192^2, N = 512 40.3 -> 37.0 us; 3000 x 6997 at 10%, N = 512 15.5 -> 13.8);
+// beyond, the panel of five workgroups a CU would lose up to 1.55x to four (bands
+// of 8192 rows, half-bandwidth 480, N = 640 22.5 against 34.5 us, the waves gain 1.17x
+// at most: 16384 x 8192 at 6%, N = 512 43.2 against 36.9).
+constexpr int kPairsMaxGroups = 1024;
+
 hipError_t run_wide(BsrArgs args, hipStream_t stream) {
     args.tiles_n = ceil_div(args.N, 64);
     const long total = static_cast<long>(ceil_div(args.block_rows, 4)) * args.tiles_n;
     if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
     args.wg_total = static_cast<int>(total);
     args.slices = record_slices(args);
-    hipLaunchKernelGGL(bsr_wide_kernel, dim3(grid_size(args)), dim3(256), 0, stream, args);
+    if (args.wg_total <= kPairsMaxGroups) {
+        hipLaunchKernelGGL(bsr_wide_kernel<true>, dim3(grid_size(args)), dim3(256), 0, stream, args);
+    } else {
+        hipLaunchKernelGGL(bsr_wide_kernel<false>, dim3(grid_size(args)), dim3(256), 0, stream, args);
+    }
     return hipGetLastError();
 }
 
@@ -1205,6 +1368,7 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
                  0,
                  0,
                  0,
+                 std::max(A.num_blocks - 8, 0) / 7,
                  1,
                  A.num_blocks,
                  reinterpret_cast<uintptr_t>(C) % 16 == 0 ? 1 : 0};
@@ -1242,18 +1406,20 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
     // structured inputs (N >= 256, 24 - 64 blocks per block-row: 1.03 - 1.31x
     // over 36 block-diagonal and banded inputs); explicit row_group 4 / 8
     // forces it.  From one block in 24 on A may as well have no structure, and
-    // then the panel takes 1.6 - 3.4 times the waves' time, so from N = 320 each
-    // launch looks (bsr_wide_kernel; against the panel: blocks at 12.5% of
-    // 8192^2, N = 512 62 -> 40 us and N = 1024 119 -> 76; 3000 x 6997 at 10%, N =
-    // 512 43 -> 14; bands and diagonal blocks within 3%), and below the waves are
-    // level on structured inputs too (12.5%, N = 256: 59 -> 19.6 us; bands 8.8 ->
-    // 8.6 and 13.4 -> 13.8, diagonal blocks of 1024 12.1 -> 8.8).  Sparser A keeps the
-    // panel: bands of 16384 rows, N = 256 take 15.0 us there, 16.8 with waves.
+    // then the panel takes 1.6 - 3.4 times the waves' time, so each launch looks
+    // (bsr_wide_kernel; against the panel: blocks at 12.5% of 8192^2, N = 512 61 ->
+    // 38 us and N = 1024 119 -> 77; 3000 x 6997 at 10%, N = 512 42 -> 14; bands and
+    // diagonal blocks 0 - 0.3 us more), except on up to one workgroup a CU: there
+    // the waves win on structured A too (bands of 4096 rows, N = 256 7.2 -> 5.0 us,
+    // diagonal blocks of 1024 11.2 -> 7.7; at 320 workgroups 12.0 against 12.5).
+    // Sparser A keeps the panel: bands of 16384 rows, N = 256 take 15.0 us there,
+    // 16.8 with waves.
     const bool panel_auto = rec && N >= 256 && A.block_cols <= kPanelMaxWords * 32 &&
                             bpr >= 24.0 && bpr <= 64.0;
     const bool dense = 24.0 * bpr >= A.block_cols;
     const bool defaults = !o.per_wave && o.row_group == 0 && o.tiles == 0 && o.depth == 0;
-    if (panel_auto && dense && defaults && N >= 320) {
+    const long panel_groups = static_cast<long>(ceil_div(A.block_rows, 4)) * ceil_div(N, 64);
+    if (panel_auto && dense && defaults && panel_groups > 256) {
         return from_hip(run_wide(args, stream), "spmm_wmma launch");
     }
     const bool panel = !o.per_wave && rec &&

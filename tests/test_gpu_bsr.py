@@ -469,3 +469,44 @@ def test_wmma_wide_b(S, O, torch, pattern, M, K, N):
     C = _run_wmma(S, torch, hb, B16.view(np.uint16))
     check_bsr(C, C32, absC)
     check_csr(C, C64, absC, tol=1e-5)
+
+
+@pytest.mark.parametrize("pattern", ["strewn", "runs", "both"])
+@pytest.mark.parametrize("M,K,N,lo,hi", [
+    (5003, 9001, 328, 26, 62),    # panel or pairs of waves in one launch: up to four workgroups a CU
+    (8501, 6007, 512, 26, 62),    # panel or waves of single blocks: more workgroups
+    (6001, 5003, 1096, 26, 62),   # the same, column tiles in slices that they do not divide
+    (2005, 12301, 256, 26, 62),   # waves alone, two tiles and four pairs in flight
+    (2005, 12301, 296, 14, 22),   # two tiles, two pairs
+    (5003, 12301, 256, 14, 22),   # four tiles, two pairs
+    (5003, 12301, 256, 97, 130),  # four tiles, four pairs
+])
+def test_wmma_strewn_or_runs(S, torch, pattern, M, K, N, lo, hi):
+    # B over 5 MiB and lo .. hi blocks per block-row: every kernel that looks at A
+    # and takes column slices or not, with row groups and tiles that the XCDs'
+    # shares do not divide and grids enlarged for the other order.
+    rng = np.random.default_rng(M + N + hi)
+    br, bc = -(-M // 16), -(-K // 16)
+    count = np.minimum(bc, lo + np.arange(br) % (hi - lo + 1))
+    row_ptr = np.concatenate([[0], count.cumsum()]).astype(np.int32)
+    cols = np.concatenate([
+        np.arange(n) + (r * 3) % (bc - n + 1) if pattern == "runs" or (pattern == "both" and r % 2)
+        else np.sort(rng.choice(bc, n, replace=False)) for r, n in enumerate(count)]).astype(np.int32)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    vals = (torch.rand((cols.size, 16, 16), generator=g, device="cuda") * 2 - 1).half()
+    rows = torch.repeat_interleave(torch.arange(br), torch.from_numpy(count)).cuda()
+    at = torch.arange(16, device="cuda")
+    c = torch.from_numpy(cols).cuda().long()
+    vals *= (rows[:, None] * 16 + at < M)[:, :, None] & (c[:, None] * 16 + at < K)[:, None, :]
+    hb = S.HostBSR(M, K, br, bc, int((vals != 0).sum()), row_ptr, cols,
+                   vals.reshape(-1).cpu().numpy().view(np.uint16))
+    B = (torch.rand((K, N), generator=g, device="cuda") * 2 - 1).half()
+    dense = torch.zeros((br, bc, 16, 16), dtype=torch.float64, device="cuda")
+    dense[rows, c] = vals.double()
+    dense = dense.transpose(1, 2).reshape(br * 16, bc * 16)[:M, :K].contiguous()
+    C64, absC = dense @ B.double(), dense.abs() @ B.double().abs()
+    say(f"wmma strewn or runs {pattern} M={M} K={K} N={N} blocks={cols.size}")
+    C = torch.full((M, N), float("nan"), device="cuda")
+    S.spmm_wmma(S.DeviceBSR(hb), B, C)
+    torch.cuda.synchronize()
+    check_csr(C.cpu().numpy(), C64.cpu().numpy(), absC.cpu().numpy(), tol=1e-5)
