@@ -1209,6 +1209,10 @@ Error from_hip(hipError_t e, const char* what) {
     return fail(kHipError, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Workgroups of 256 threads: HIP 7.0 takes a launch of 2^32 threads and more without
+// an error and runs none or a part of it.
+constexpr long kMaxGroups = 0xffffffffL / 256;
+
 // B rows and A blocks fit structured-buffer records: the record stride field
 // holds at most 16383 bytes and each buffer must stay within 2 GiB.
 bool records_fit(const BsrArgs& a) {
@@ -1245,14 +1249,20 @@ unsigned grid_size(const BsrArgs& a) {
     return std::max(sliced, static_cast<unsigned>(a.wg_total));
 }
 
+// Sets the column slices of tiles_n and wg_total and returns the grid.
+unsigned slice_grid(BsrArgs& a) {
+    a.slices = record_slices(a);
+    if (grid_size(a) > kMaxGroups) a.slices = 1;
+    return grid_size(a);
+}
+
 template <int J, int D>
 hipError_t run_wave(BsrArgs args, hipStream_t stream, bool pointer_addressing) {
     args.tiles_n = ceil_div(args.N, 16 * J);
     const long total = static_cast<long>(ceil_div(args.block_rows, 4)) * args.tiles_n;
-    if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
+    if (total > kMaxGroups) return hipErrorInvalidConfiguration;
     args.wg_total = static_cast<int>(total);
-    args.slices = record_slices(args);
-    const unsigned tiles = grid_size(args);
+    const unsigned tiles = slice_grid(args);
     if (!pointer_addressing && records_fit(args)) {
         hipLaunchKernelGGL((bsr_record_kernel<J, D == 1 ? 2 : D>), dim3(tiles), dim3(256), 0,
                            stream, args);
@@ -1282,7 +1292,7 @@ template <int R, int J, int WR, int D>
 hipError_t run_panel(BsrArgs args, hipStream_t stream) {
     args.tiles_n = ceil_div(args.N, 16 * J);
     const long total = static_cast<long>(ceil_div(args.block_rows, R)) * args.tiles_n;
-    if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
+    if (total > kMaxGroups) return hipErrorInvalidConfiguration;
     args.wg_total = static_cast<int>(total);
     hipLaunchKernelGGL((bsr_panel_kernel<R, J, WR, D>), dim3(args.wg_total), dim3(256), 0, stream,
                        args);
@@ -1300,13 +1310,13 @@ constexpr int kPairsMaxGroups = 1024;
 hipError_t run_wide(BsrArgs args, hipStream_t stream) {
     args.tiles_n = ceil_div(args.N, 64);
     const long total = static_cast<long>(ceil_div(args.block_rows, 4)) * args.tiles_n;
-    if (total > 0x7fffffffL) return hipErrorInvalidConfiguration;
+    if (total > kMaxGroups) return hipErrorInvalidConfiguration;
     args.wg_total = static_cast<int>(total);
-    args.slices = record_slices(args);
+    const unsigned grid = slice_grid(args);
     if (args.wg_total <= kPairsMaxGroups) {
-        hipLaunchKernelGGL(bsr_wide_kernel<true>, dim3(grid_size(args)), dim3(256), 0, stream, args);
+        hipLaunchKernelGGL(bsr_wide_kernel<true>, dim3(grid), dim3(256), 0, stream, args);
     } else {
-        hipLaunchKernelGGL(bsr_wide_kernel<false>, dim3(grid_size(args)), dim3(256), 0, stream, args);
+        hipLaunchKernelGGL(bsr_wide_kernel<false>, dim3(grid), dim3(256), 0, stream, args);
     }
     return hipGetLastError();
 }

@@ -1277,6 +1277,21 @@ int pick_vec(int N, int want) {
     return want;
 }
 
+// Threads of a launch.  HIP 7.0 takes a launch of 2^32 and more without an error
+// and runs none or a part of it.
+constexpr long kMaxThreads = 0xffffffffL;
+
+Error check_threads(long grid, int threads) {
+    if (grid * threads <= kMaxThreads) return ok();
+    return fail(kUnsupported, "the launch would need 2^32 threads or more");
+}
+
+// Workgroups of nblocks row blocks in column slices (see the kernels).
+long sliced_grid(long nblocks, int slices) {
+    const int per = 8 / slices;
+    return slices == 1 ? nblocks : (nblocks + per - 1) / per * 8;
+}
+
 // Lane groups of a wave: with L = lanes of one row (slice) and p column passes
 // a group takes ceil(L / p) lanes; the pass count with the fewest passes per
 // entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
@@ -1532,9 +1547,16 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
     if (o.row_groups == 2) coop = false;
     else if (o.row_groups == 3) coop = true;
     else coop = lc_log >= 2 && (avg >= 32.0 || (static_cast<long>(M) << lc_log) >= (1L << 18));
-    const int rows_per_wg = 4 * (kWave >> (lc_log + le_log));
-    const int nblocks = ceil_div(M, rows_per_wg);
-    const int grid = slices == 1 ? nblocks : ceil_div(nblocks, 8 / slices) * 8;
+    // Entry lanes that no cap holds down may be more than a launch has threads
+    // for (17 M rows of 20, N = 132 in eight slices of five column lanes).
+    const auto blocks_of = [&](int le) { return ceil_div(M, 4 * (kWave >> (lc_log + le))); };
+    while (o.entry_lanes == 0 && le_log > 0 &&
+           sliced_grid(blocks_of(le_log), slices) * 256 > kMaxThreads) {
+        --le_log;
+    }
+    const int nblocks = blocks_of(le_log);
+    if (Error e = check_threads(sliced_grid(nblocks, slices), 256); e.status != kOk) return e;
+    const int grid = static_cast<int>(sliced_grid(nblocks, slices));
     const int long_len = std::max(8 << le_log << (unroll == 4 ? 2 : 1),
                                   static_cast<int>(std::ceil(std::min(4.0 * avg, 1.0e9))));
     RowGroupArgs args{A.row_ptr, A.col_idx,  A.values,   B,          C,
@@ -1551,22 +1573,30 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
 }
 
 // Column lanes: the fewest (a power of two, at most 64) that cover N; wider N in
-// column tiles of 256, a workgroup each.
+// column tiles of 256, a workgroup each.  Rows past a launch's threads (67 M at 64
+// lanes) go into further launches.
 Error launch_in_order(const CSR& A, const float* B, float* C, int N, hipStream_t stream) {
-    const int vec    = pick_vec(N, 0);
-    const int lc_log = pow2_log_at_least(ceil_div(N, vec));
-    const dim3 grid(ceil_div(A.num_rows, 4 * (kWave >> lc_log)),
-                    std::min(ceil_div(N, vec << lc_log), 65535));
-    const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, A.num_rows, N, lc_log, A.row_ptr,
-                           A.col_idx, A.values, B, C);
-        return from_hip(hipGetLastError(), "csr in-order launch");
-    };
-    if (vec == 1) return run(csr_rows_in_order<1, Hand::Direct>);
-    if (vec == 2) return run(csr_rows_in_order<2, Hand::Direct>);
-    if (lc_log == 6) return run(csr_rows_in_order<4, Hand::Readlane>);
-    return lc_log >= 3 ? run(csr_rows_in_order<4, Hand::Shuffle>)
-                       : run(csr_rows_in_order<4, Hand::Direct>);
+    const int  vec    = pick_vec(N, 0);
+    const int  lc_log = pow2_log_at_least(ceil_div(N, vec));
+    const int  per_wg = 4 * (kWave >> lc_log);
+    const long most   = kMaxThreads / 256 * per_wg;
+    for (long first = 0; first < A.num_rows; first += most) {
+        const int  rows = static_cast<int>(std::min(most, A.num_rows - first));
+        const dim3 grid(ceil_div(rows, per_wg), std::min(ceil_div(N, vec << lc_log), 65535));
+        const auto run = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, rows, N, lc_log,
+                               A.row_ptr + first, A.col_idx, A.values, B,
+                               C + static_cast<size_t>(first) * N);
+            return from_hip(hipGetLastError(), "csr in-order launch");
+        };
+        const Error e = vec == 1      ? run(csr_rows_in_order<1, Hand::Direct>)
+                        : vec == 2    ? run(csr_rows_in_order<2, Hand::Direct>)
+                        : lc_log == 6 ? run(csr_rows_in_order<4, Hand::Readlane>)
+                        : lc_log >= 3 ? run(csr_rows_in_order<4, Hand::Shuffle>)
+                                      : run(csr_rows_in_order<4, Hand::Direct>);
+        if (e.status != kOk) return e;
+    }
+    return ok();
 }
 
 Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int N,
@@ -1701,15 +1731,26 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
             rpb = std::min(rpb, M / (slices == 1 ? 512 : 256));
         }
         rpb = std::max(1, std::min(rpb, kRpCap));
+        // 160 entries per wave in eight slices are more threads than a launch
+        // has from 1.3 G entries on.
+        while (o.rows_per_block <= 0 && rpb < kRpCap &&
+               sliced_grid(ceil_div(M, rpb), slices) * (waves * kWave) > kMaxThreads) {
+            rpb = std::min(2 * rpb, kRpCap);
+        }
         args.rows_per_block = rpb;
         part.nblocks = ceil_div(M, rpb);
     }
-    const int grid = slices == 1 ? part.nblocks : ceil_div(part.nblocks, 8 / slices) * 8;
-    hipError_t e;
     const bool balanced = even || split != nullptr;
-    if (balanced && sbuf && vec == 4 && args.groups <= 2 && o.groups == 0 && o.waves == 0 &&
-        o.unroll == 0) {
-        e = dispatch_wide<false>(even || slices > 1 ? 4 : 8, args, grid, stream);
+    const bool wide = balanced && sbuf && vec == 4 && args.groups <= 2 && o.groups == 0 &&
+                      o.waves == 0 && o.unroll == 0;
+    const int wg_waves = !sbuf ? 8 : wide ? (even || slices > 1 ? 4 : 8) : waves;
+    if (Error t = check_threads(sliced_grid(part.nblocks, slices), wg_waves * kWave); t.status != kOk) {
+        return t;
+    }
+    const int grid = static_cast<int>(sliced_grid(part.nblocks, slices));
+    hipError_t e;
+    if (wide) {
+        e = dispatch_wide<false>(wg_waves, args, grid, stream);
     } else if (vec == 4) {
         e = dispatch_shape<4>(waves, unroll, sbuf, args, grid, stream);
     } else if (vec == 2) {

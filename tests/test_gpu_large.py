@@ -197,3 +197,39 @@ def test_large_khalf(S, torch):
         diff = (C12 - (C1 + C2)).abs().max().item()
         scale = C12.abs().max().item()
         assert diff <= 1e-5 * max(scale, 1.0) * 64, (diff, scale)
+
+
+def _same_rows(S, torch, M, K, per):
+    """Device CSR whose rows all hold the same columns with values of one, made
+    on the device; (matrix, the columns)."""
+    cols = torch.arange(per, device="cuda", dtype=torch.int32) * (K // per)
+    A = S.DeviceCSR.__new__(S.DeviceCSR)
+    A.num_rows, A.num_cols, A.nnz = M, K, M * per
+    A.row_ptr = torch.arange(M + 1, device="cuda", dtype=torch.int32) * per
+    A.col_idx = cols.repeat(M)
+    A.values = torch.ones(M * per, dtype=torch.float32, device="cuda")
+    return A, cols.long()
+
+
+@pytest.mark.parametrize("form,M,K,per,N", [
+    # More than 2^32 threads at the entry lanes, rows per workgroup or one launch that
+    # smaller matrices take: 32 lanes a row in eight slices; one row per workgroup of four
+    # waves in eight slices; 64 lanes a row.
+    ("groups", 17_000_000, 4096, 20, 132),
+    ("engine", 2_200_000, 20000, 430, 256),
+    ("baseline", 67_200_000, 64, 1, 129),
+    ("memopt_v2", 67_200_000, 64, 1, 129),
+])
+def test_more_threads_than_a_launch_holds(S, torch, form, M, K, per, N):
+    say(f"large csr {form} {M} x {K}, {per} per row, N={N}")
+    A, cols = _same_rows(S, torch, M, K, per)
+    B = (torch.arange(K * N, device="cuda") % 251 - 125).float().view(K, N)
+    want = B[cols].double().sum(0).float()  # whole numbers below 2^24: exact in any order
+    C = torch.full((M, N), float("nan"), device="cuda")
+    if form == "groups":
+        S.spmm_tiled_v3_opts(A, B, S.EngineOptsT(row_groups=1, slices=8), C)
+    else:
+        S.spmm_csr("tiled_v3" if form == "engine" else form, A, B, C)
+    torch.cuda.synchronize()
+    for i in range(0, M, 1 << 20):
+        assert (C[i:i + (1 << 20)] == want).all(), i
