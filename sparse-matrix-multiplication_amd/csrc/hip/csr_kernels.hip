@@ -1367,16 +1367,16 @@ hipError_t dispatch_wide(int waves, const RowblockArgs& args, int grid, hipStrea
 // through too.  Measured on MI355X over 70 uniform and power-law inputs with B
 // of 8 .. 256 MiB, against slices of at least 64 columns: 65536^2, 32 per row,
 // N = 256 252 -> 212 us; 32768^2, 32 per row, N = 128 46.7 -> 38.9 us; 8192^2, 100
-// per row, N = 512 70 -> 64 us.  B of 4 MiB or less is fastest unsliced.  Rows
-// that are no whole number of lines keep 64 columns: every slice of such a row
-// touches one line more (131072^2, 8 per row, N = 500: 414 us with 4 slices, 447
-// with 8).
+// per row, N = 512 70 -> 64 us.  B of 4 MiB or less is fastest unsliced.  Slices
+// that are no whole number of lines keep 64 columns: every one touches a line
+// more (131072^2, 8 per row, N = 500: 414 us with 4 slices, 447 with 8; 65536^2, 32
+// per row, N = 96 99 us whole, 131 with 2; N = 192 226 with 2, 263 with 4).
 int auto_slices(int K, int N, double avg_row) {
     const long long b_bytes = static_cast<long long>(K) * N * 4;
     if (b_bytes <= (4LL << 20)) return 1;
-    const int narrowest = N % 32 == 0 ? 32 : 64;
+    const auto narrowest = [&](int slices) { return N % (32 * slices) == 0 ? 32 : 64; };
     int s = 1;
-    while (s < 8 && ((b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest) ||
+    while (s < 8 && ((b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest(2 * s)) ||
                      (b_bytes > (2LL << 20) * s && N / (2 * s) >= 64 && avg_row >= 16.0))) {
         s *= 2;
     }
@@ -1823,7 +1823,7 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     // (24576^2, 100 per row, N = 100 65 against 99 us; over 90 inputs with N = 33
     // .. 250 they lose at most 3%, and at N = 250 on rows of 24 and fewer 15%).
     const double b_mib = static_cast<double>(K) * N / (1 << 18);
-    const bool lines = N % 32 == 0;
+    const bool lines = N % (N <= 128 ? 64 : 32) == 0;  // N = 96 has no halves of whole lines
     if (N <= 32 && K > 98304 && avg_row >= 16.0) return false;
     if (lines && N > 32 && N <= 64 && b_mib >= 16.0) return false;
     if (lines && N > 64 && b_mib > 4.0 &&

@@ -241,6 +241,12 @@ def test_bsr_stats_from_csr_host_equals_full_build(S):
             assert getattr(fast, f) == getattr(full, f), f
 
 
+def _even_rows(S, M, K, per):
+    """A host CSR of equal rows; the columns are all 0 (the form reads lengths)."""
+    return S.HostCSR(M, K, np.arange(M + 1, dtype=np.int32) * per, np.zeros(M * per, np.int32),
+                     np.ones(M * per, np.float32))
+
+
 def test_csr_auto_form(S):
     # the CSR form spmm_hybrid_run picks from the row lengths (host only):
     # row groups, the engine with the longest row as hint, or merge-path
@@ -279,6 +285,12 @@ def test_csr_auto_form(S):
     assert longest(pl) <= 512
     assert S.csr_auto_form(pl, 128)[0] == "engine"
     assert S.csr_auto_form(pl, 16)[0] == "rowgroups"
+    # N = 96 cannot be cut into slices of whole 128-byte lines as N = 64 and 128
+    # can, with which the engine wins on a B past the L2s
+    assert [S.csr_auto_form(_even_rows(S, 24576, 24576, 100), n)[0] for n in (64, 96, 128)] == [
+        "rowgroups", "rowgroups", "engine"]
+    assert [S.csr_auto_form(_even_rows(S, 65536, 65536, 40), n)[0] for n in (64, 96, 128)] == [
+        "engine", "rowgroups", "engine"]
     # no nonzeros: the engine, no hint
     empty = S.csr_from_coo_host(8, 8, [], [], [])
     assert S.csr_auto_form(empty, 32)[:2][0] == "engine"
