@@ -1485,20 +1485,41 @@ hipError_t run_row_groups(const RowGroupArgs& args, bool coop, bool long_rows, i
                 : run_row_groups<VEC, false, false>(args, unroll, grid, stream);
 }
 
+// Whether rows take their entry lanes past the cap that keeps the grid near 8192
+// waves.  Long rows of narrow B are bound by one 128-byte line per entry into the
+// L1s (262144 rows of 24, N = 1: 6.3 M lines in 31 us, 26 TB/s, where gathers
+// saturate), and a lane that walks much of a row alone also takes a line of
+// col_idx and of values per step.  le_log: the capped lanes.  MI355X, capped
+// against uncapped (M = K, uniform rows unless said):
+//  - up to 2 column lanes from 10 entries per lane on (49152 rows of 80, N = 8 26.3
+//    -> 21.8 us; 20000 of 60 at 7.5 per lane 13.3 -> 14.0), from 49152 rows on from 5
+//    (98304 rows of 24, N = 1 13.3 -> 12.5; 262144 45.3 -> 30.6);
+//  - at 4 from 11 (24576 rows of 80, N = 16 12.9 -> 12.3; of 40, 10 per lane, 7.6 -> 7.8);
+//  - at 8 where B is past the L2s (65536 rows of 40, N = 32 37.0 -> 33.5; 49152 rows, a
+//    B of 6 MiB, 21.1 -> 23.5), on rows of 128 and more (32768 of 160 39.1 -> 37.2),
+//    and on uneven rows (power-law 32768 of 76 58 -> 39); without a longest-row
+//    hint, which would tell, on rows of 64 and more of a B in an L2 (24576 of 80
+//    16.0 -> 16.4);
+//  - not from 16 column lanes on, nor on rows of under 20.
+bool more_entry_lanes(int M, int K, int N, long long nnz, int max_row, int lc_log, int le_log) {
+    const double avg = static_cast<double>(nnz) / M;
+    const double per_lane = avg / (1 << le_log);
+    if (avg < 20.0 || lc_log > 3) return false;
+    if (lc_log <= 1) return per_lane >= (M >= 49152 ? 5.0 : 10.0);
+    if (lc_log == 2) return per_lane >= 11.0;
+    const long long b_bytes = static_cast<long long>(K) * N * 4;
+    if (avg >= 128.0 || b_bytes >= (8LL << 20)) return true;
+    return max_row > 0 ? !rows_even(M, nnz, max_row) : avg >= 64.0 && b_bytes <= (4LL << 20);
+}
+
 // Shape of the sub-wave row groups, measured on MI355X over uniform rows of
 // 1 .. 300 entries, M = 2048 .. 65536 and N = 1 .. 256:
 //  - column lanes cover N in one pass (up to 64 lanes), except that 32 or 64
 //    column lanes drop to 16 (two or four passes) while the matrix would
 //    still give >= 16384 waves (e.g. M = 32768, N = 128: 96 -> 89 us);
-//  - entry lanes ~1.5 * sqrt(average row) as a power of two (sqrt from 4 column
-//    lanes on), but on rows of under 20 entries, or from 16 column lanes on, no
-//    more than keep the grid near 8192 waves (32 per CU): beyond that, more
-//    rows per wave beat more lanes per row.  Longer rows of narrow B are bound
-//    by one 128-byte line per entry into the L1s (262144 rows of 24, N = 1: 6.3 M
-//    lines in 31 us, 26 TB/s, where gathers saturate), and a lane that walks a
-//    row alone also takes a line of col_idx and of values per step: 45 -> 31 us
-//    there, 131072 rows of 120, N = 8 168 -> 96 us; of 3 at N = 32 12.3 against 13.4
-//    with two lanes instead of one;
+//  - entry lanes ~1.5 * sqrt(average row) as a power of two, but no more than
+//    keep the grid near 8192 waves (32 per CU): beyond that, more rows per wave
+//    beat more lanes per row -- except on the rows of more_entry_lanes;
 //  - 4 entries per entry lane per iteration on those, and from 32 entries per
 //    row on while B is at most 2 MiB (latency-bound: few, long rows), else 2 -- with B
 //    beyond one XCD's L2, fewer gathers in flight keep more of it cached
@@ -1521,28 +1542,32 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     const int slice_cols = ceil_div(ceil_div(N, slices), vec) * vec;
     const int lc_log = row_group_lc_log(M, slice_cols, vec);
-    const bool deep = avg >= 20.0 && lc_log <= 3;
     int le_log;
+    bool more = false;
     if (o.entry_lanes != 0) {
         if (o.entry_lanes < 0 || o.entry_lanes > 64 || (o.entry_lanes & (o.entry_lanes - 1)) != 0) {
             return fail(kInvalid, "entry_lanes must be a power of two up to 64");
         }
         le_log = pow2_log_at_least(o.entry_lanes);
     } else {
-        const double want = (deep && lc_log >= 2 ? 1.0 : 1.5) * std::sqrt(std::max(avg, 1.0));
-        le_log = static_cast<int>(std::lround(std::log2(want)));
-        if (!deep) {
-            const long cap =
-                kTargetWaves * kWave / std::max(1L, (static_cast<long>(M) << lc_log) * slices);
-            int cap_log = 0;
-            while ((2L << cap_log) <= cap) ++cap_log;
-            le_log = std::min(le_log, cap_log);
-        }
+        // Lanes by row length; fewer suffice at 4 column lanes and more.
+        const auto lanes_for = [&](double factor) {
+            return static_cast<int>(std::lround(std::log2(factor * std::sqrt(std::max(avg, 1.0)))));
+        };
+        const long cap =
+            kTargetWaves * kWave / std::max(1L, (static_cast<long>(M) << lc_log) * slices);
+        int cap_log = 0;
+        while ((2L << cap_log) <= cap) ++cap_log;
+        le_log = std::max(0, std::min(lanes_for(1.5), cap_log));
+        const int long_log = std::min(lanes_for(lc_log >= 2 ? 1.0 : 1.5), 6 - lc_log);
+        more = long_log > le_log &&
+               more_entry_lanes(M, A.num_cols, N, A.nnz, o.max_row_hint, lc_log, le_log);
+        if (more) le_log = long_log;
     }
     le_log = std::max(0, std::min(le_log, 6 - lc_log));
     const bool b_small = static_cast<long long>(A.num_cols) * N * 4 <= (2LL << 20);
     const int unroll = (o.unroll == 2 || o.unroll == 4) ? o.unroll
-                                                        : (deep || (avg >= 32.0 && b_small) ? 4 : 2);
+                                                        : (more || (avg >= 32.0 && b_small) ? 4 : 2);
     bool coop;
     if (o.row_groups == 2) coop = false;
     else if (o.row_groups == 3) coop = true;

@@ -629,3 +629,26 @@ def test_engine_rounding(S, O, torch, N):
         # One or two groups on merge-path parts take alternate entries instead:
         # two chains, or one per row at N over 128.
         assert rel <= bound * (1.5 if name == "split" and N == 100 else 1.0), (name, rel, bound)
+
+
+def test_row_groups_rounding(S, O, torch):
+    # Rows of 80 at N = 16: sixteen entry lanes, whose chains are added pairwise.
+    # The same sums in fp32 on the CPU give the error; fewer lanes have longer
+    # chains (eight: 9% more).  1.04: the order inside a chain may differ.
+    M, K, per, N = 2000, 1500, 80, 16
+    rng = np.random.default_rng(6)
+    col = np.sort(rng.random((M, K)).argpartition(per, 1)[:, :per], 1).astype(np.int32)
+    val = rng.uniform(-1, 1, (M, per)).astype(np.float32)
+    A = S.HostCSR(M, K, np.arange(M + 1, dtype=np.int32) * per, col.ravel(), val.ravel())
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    C64, absC = O.csr_spmm_f64(A.row_ptr, A.col_idx, A.values, B)
+    part = np.zeros((16, M, N), np.float32)
+    for e in range(per):  # a product of fp32 is exact in fp64: one rounding, as a fused step
+        part[e % 16] = (val[:, e, None].astype(np.float64) * B[col[:, e]] + part[e % 16]).astype(np.float32)
+    while len(part) > 1:
+        part = part[0::2] + part[1::2]
+    bound = 1.04 * np.linalg.norm(part[0] - C64) / np.linalg.norm(C64)
+    say(f"csr row groups rounding N={N}")
+    C = S.spmm_csr("tiled_v3", S.DeviceCSR(A), torch.from_numpy(B).cuda()).cpu().numpy()
+    rel = check_csr(C, C64, absC)
+    assert rel <= bound, (rel, bound)
