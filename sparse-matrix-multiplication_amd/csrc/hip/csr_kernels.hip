@@ -1849,8 +1849,17 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     // .. 250 they lose at most 3%, and at N = 250 on rows of 24 and fewer 15%).
     const double b_mib = static_cast<double>(K) * N / (1 << 18);
     const bool lines = N % (N <= 128 ? 64 : 32) == 0;  // N = 96 has no halves of whole lines
-    if (N <= 32 && K > 98304 && avg_row >= 16.0) return false;
-    if (lines && N > 32 && N <= 64 && b_mib >= 16.0) return false;
+    // Narrow B and rows just too short for more_entry_lanes, on many rows with a B
+    // past the L2s (or so many that the lines of A alone bound a lane per row):
+    // 262144 x 400000, 17 per row, N = 8 90 against 66 us, 500000 x 131072, N = 1 72
+    // against 62; 131072 x 400000, N = 4 26.5 against 30.4, 262144 x 131072, N = 4 34
+    // against 49, 20000 x 131072, N = 1 3.8 against 7.4 (over 180 shapes of 16 to 19 per
+    // row; longer rows: 262144^2, 24 per row, N = 1 31 against 42, N = 16 97 against 95).
+    if (N <= 32 && avg_row >= 16.0 && avg_row < 20.0 &&
+        ((M >= 131072 && b_mib > 4.0 && b_mib * M >= 8.0 * 131072) || (M >= 400000 && K > 65536))) {
+        return false;
+    }
+    if (lines && N > 32 && N <= 64 && b_mib >= 16.0 && avg_row >= 16.0) return false;
     if (lines && N > 64 && b_mib > 4.0 &&
         (avg_row >= (N > 128 ? 16.0 : 24.0) || (N <= 128 && b_mib >= 32.0))) {
         return false;

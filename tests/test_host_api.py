@@ -291,6 +291,15 @@ def test_csr_auto_form(S):
         "rowgroups", "rowgroups", "engine"]
     assert [S.csr_auto_form(_even_rows(S, 65536, 65536, 40), n)[0] for n in (64, 96, 128)] == [
         "engine", "rowgroups", "engine"]
+    # narrow B: rows of 20 and more take more entry lanes, shorter ones leave many
+    # rows with a B past the L2s to the engine
+    forms = lambda m, ns: [S.csr_auto_form(m, n)[0] for n in ns]
+    for m in (_even_rows(S, 131072, 131072, 24), _even_rows(S, 20000, 200000, 60),
+              _even_rows(S, 20000, 131072, 17), _even_rows(S, 99000, 99000, 17)):
+        assert forms(m, (1, 4, 8, 16, 32)) == ["rowgroups"] * 5
+    assert forms(_even_rows(S, 262144, 131072, 17), (1, 4, 16, 32)) == [
+        "rowgroups", "rowgroups", "engine", "engine"]
+    assert forms(_even_rows(S, 400000, 131072, 17), (1, 8)) == ["engine"] * 2
     # no nonzeros: the engine, no hint
     empty = S.csr_from_coo_host(8, 8, [], [], [])
     assert S.csr_auto_form(empty, 32)[:2][0] == "engine"
