@@ -1452,13 +1452,20 @@ int row_group_lc_log(int M, int N, int vec) {
 // 4 MiB (measured on MI355X: M = 16384, N = 256, 16 per row 28.4 -> 20.2 us
 // with 4 slices; M = 32768, N = 128: 28.5 -> 25.0 us).  Longer rows keep one
 // slice: every slice re-reads the rows' column indices, which then costs more
-// than the L2 misses it saves.
+// than the L2 misses it saves.  Widths that are no whole lines take slices only
+// where wide ones (64 columns, 48 from four slices on) do bring the share down,
+// to 6 MiB: every slice touches a line more (M = 16384, 16 per row, N = 500 64 us
+// with four slices, 54 with eight; N = 250 33 with two, 29 with four; M = 65536, N =
+// 250 168 whole, 211 with two; N = 100 66 whole, 83 with two).
 int row_group_slices(int K, int N, double avg_row) {
     if (avg_row > 24.0) return 1;
     const long long b_bytes = static_cast<long long>(K) * N * 4;
-    const int narrowest = N % 32 == 0 ? 32 : 64;  // whole lines, as in auto_slices
     int s = 1;
-    while (s < 8 && b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest) s *= 2;
+    if (N % 32 != 0) {
+        while (s < 8 && b_bytes > (6LL << 20) * s) s *= 2;
+        return b_bytes <= (6LL << 20) * s && N / s >= (s == 2 ? 64 : 48) ? s : 1;
+    }
+    while (s < 8 && b_bytes > (4LL << 20) * s && N / (2 * s) >= 32) s *= 2;
     return s;
 }
 
@@ -1823,8 +1830,8 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     // the engine with the longest row as its hint; power-law rows capped at
     // 512 / 4096).  Row groups win 1.5 - 4x for N <= 32 and 1.1 - 1.7x for
     // N = 64 (not on 1024 rows of > 100 entries, 0.75 - 0.9x).  Above
-    // N = 64 they win on short rows (N x average <= 4096), when B needs
-    // column slices, and at N = 128 on >= 4096 rows (1.03 - 1.6x) or >= 2048
+    // N = 64 they win on short rows (N x average <= 4096), on rows of up to 24
+    // entries of a B past an L2, and at N = 128 on >= 4096 rows (1.03 - 1.6x) or >= 2048
     // rows of up to 10600 / N entries -- except at 4097 .. 8192 rows of
     // >= 64 entries, where the engine's whole-round grid holds 1 - 2 rows
     // per wave and matches or beats them (0.97 - 1.00x).  Those wins need
@@ -1865,7 +1872,8 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
         return false;
     }
     if (N <= 64) return M >= 2048 || avg_row <= 100.0;
-    if (N * avg_row <= 2048.0 || (N <= 256 && slices > 1)) return true;
+    const bool b_large = avg_row <= 24.0 && b_mib > 4.0 && N >= (N % 32 == 0 ? 64 : 128);
+    if (N * avg_row <= 2048.0 || (N <= 256 && b_large)) return true;
     if (max_row > 2.0 * avg_row + 32.0) return false;  // uneven rows
     if (!lines && N <= 256 && b_mib > 4.0) return true;
     if (N * avg_row <= 4096.0) return true;

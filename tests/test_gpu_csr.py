@@ -652,3 +652,18 @@ def test_row_groups_rounding(S, O, torch):
     C = S.spmm_csr("tiled_v3", S.DeviceCSR(A), torch.from_numpy(B).cuda()).cpu().numpy()
     rel = check_csr(C, C64, absC)
     assert rel <= bound, (rel, bound)
+
+
+@pytest.mark.parametrize("N", [100, 130, 198, 250, 499, 512])
+def test_row_groups_column_slices(S, O, torch, N):
+    # B past an L2 under rows of up to 24: whole, or in two to eight slices whose
+    # columns are no whole number of lanes, lines or slices.
+    A = S.generate_uniform_random_csr(700, 17001, 10 / 17001, 23)
+    B = np.random.default_rng(N).uniform(-1, 1, (A.num_cols, N)).astype(np.float32)
+    C64, absC = O.csr_spmm_f64(A.row_ptr, A.col_idx, A.values, B)
+    dA, dB = S.DeviceCSR(A), torch.from_numpy(B).cuda()
+    say(f"csr row groups slices N={N}")
+    C = torch.full((A.num_rows, N), float("nan"), device="cuda")
+    S.spmm_tiled_v3_opts(dA, dB, S.EngineOptsT(row_groups=1), C)
+    torch.cuda.synchronize()
+    check_csr(C.cpu().numpy(), C64, absC)
