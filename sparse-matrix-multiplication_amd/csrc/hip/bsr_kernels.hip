@@ -178,7 +178,14 @@ __device__ __forceinline__ f16x8 drop_low(f16x8 v, int n) {
     return __builtin_bit_cast(f16x8, n < 8 ? x >> (16 * n) : static_cast<unsigned __int128>(0));
 }
 
-template <int J, int D, bool VEC>
+// How a lane gets its eight elements of a B row: one at a time (B smaller than a
+// chunk), 16 bytes at any element, or 16 bytes at a 16-byte address of rows
+// that are whole chunks.  The last needs neither end of B nor shift: 3 - 30% less
+// time than the any-element form there (32768^2 diagonal blocks of 256, N = 32 4.8
+// against 6.8 us; 8192^2 blocks at 12.5%, N = 64 11.2 against 13.9).
+enum class Chunks { Elements, Any, Aligned };
+
+template <int J, int D, Chunks B_CHUNKS>
 __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
     constexpr int NT  = 16 * J;          // columns per wave
     constexpr int S   = NT + 16;         // LDS row stride in fp16 (S/2 = 8 mod 32 banks)
@@ -231,7 +238,11 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
             const int n   = n0 + (idx % CH) * 8;
             const bool ok = (s < 16 || two) && k < a.K && n < a.N;
             r.b_ok[c] = ok;
-            if constexpr (VEC) {
+            if constexpr (B_CHUNKS == Chunks::Aligned) {
+                const size_t off = ok ? static_cast<size_t>(k) * a.N + n : 0;
+                r.shift[c] = 0;
+                r.b[c] = *reinterpret_cast<const f16x8*>(a.B + off);
+            } else if constexpr (B_CHUNKS == Chunks::Any) {
                 // A row may start at any element (Mem) and the last chunk of a
                 // row may run into the next row: those products land in output
                 // columns >= N, which are never stored.  Only past the end of
@@ -265,7 +276,7 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
             const int idx = lane + c * 64;
             const f16x8 zero = f16x8(static_cast<_Float16>(0.0f));
             f16x8 b = r.b[c];
-            if constexpr (VEC) {
+            if constexpr (B_CHUNKS == Chunks::Any) {
                 if (__builtin_expect(__any(r.shift[c] != 0), 0)) b = drop_low(b, r.shift[c]);
             }
             *reinterpret_cast<f16x8*>(&tile[(idx / CH) * S + (idx % CH) * 8]) =
@@ -1268,13 +1279,16 @@ hipError_t run_wave(BsrArgs args, hipStream_t stream, bool pointer_addressing) {
                            stream, args);
         return hipGetLastError();
     }
-    if (static_cast<long long>(args.K) * args.N >= 8) {
-        hipLaunchKernelGGL((bsr_wave_kernel<J, D, true>), dim3(args.wg_total), dim3(256), 0,
+    if (args.b_vec_ok) {
+        hipLaunchKernelGGL((bsr_wave_kernel<J, D, Chunks::Aligned>), dim3(args.wg_total), dim3(256),
+                           0, stream, args);
+    } else if (static_cast<long long>(args.K) * args.N >= 8) {
+        hipLaunchKernelGGL((bsr_wave_kernel<J, D, Chunks::Any>), dim3(args.wg_total), dim3(256), 0,
                            stream, args);
     } else {  // B is smaller than one chunk
         args.tiles_n  = 1;
         args.wg_total = ceil_div(args.block_rows, 4);
-        hipLaunchKernelGGL((bsr_wave_kernel<1, 1, false>), dim3(args.wg_total), dim3(256), 0,
+        hipLaunchKernelGGL((bsr_wave_kernel<1, 1, Chunks::Elements>), dim3(args.wg_total), dim3(256), 0,
                            stream, args);
     }
     return hipGetLastError();
@@ -1459,13 +1473,17 @@ Error launch_bsr(const BSR& A, const half* B, float* C, int N, hipStream_t strea
     // stages through registers: four tiles pay from 2048 waves on, with one
     // pair in flight (8192^2 blocks at 12.5%, N = 500: 46 us against 75 with two
     // tiles and 52 with two pairs; at 1024 waves 52 against 35), and one tile
-    // below 512 waves of two (2000^2, N = 36: 4.1 against 5.1 us).
+    // below 512 waves of two (2000^2, N = 36: 4.1 against 5.1 us).  Where its chunks
+    // are aligned four tiles need N >= 256 and 12 blocks per block-row besides
+    // (8192^2 at 12.5%, N = 512 73 -> 42 us; N = 128 15.2 against 24, bands of 5 blocks,
+    // N = 256 6.4 against 7.1).
     const long waves4 = static_cast<long>(A.block_rows) * ((N + 63) / 64);
     const long waves2 = static_cast<long>(A.block_rows) * ((N + 31) / 32);
+    const bool ptr4 = waves4 >= 2048 && (!args.b_vec_ok || (N >= 256 && bpr >= 12.0));
     const int j_auto =
         N <= 16 ? 1
         : rec   ? ((waves4 >= 1024 && (bpr >= 12.0 || waves4 >= 2048)) ? 4 : 2)
-                : (waves4 >= 2048 ? 4 : (waves2 >= 512 ? 2 : 1));
+                : (ptr4 ? 4 : (waves2 >= 512 ? 2 : 1));
     const int j = (o.tiles == 1 || o.tiles == 2 || o.tiles == 4) ? o.tiles : j_auto;
     const int d_auto = rec ? (bpr >= (j == 4 ? 96.0 : 30.0) ? 4 : 2) : (j == 4 ? 1 : 2);
     const int d = (o.depth == 1 || o.depth == 2 || o.depth == 4) ? o.depth : d_auto;
