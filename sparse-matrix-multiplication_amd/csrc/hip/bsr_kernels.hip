@@ -122,10 +122,12 @@ struct RunSample {
 // that neighbouring block-rows share are fetched into one L2 only.
 // With S > 1 slices, XCDs s*8/S .. (s+1)*8/S - 1 take the s-th part of the
 // column tiles, each a band of the block-rows: its L2 holds 1/S of B.
+// ONE: one slice and a grid of just the tiles.
+template <bool ONE = false>
 __device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int slices, int& bx, int& by) {
     const int L = blockIdx.x;
     const int xcd = L & 7, idx = L >> 3;
-    if (slices > 1) {
+    if (!ONE && slices > 1) {
         const int bands = 8 / slices;
         const int tiles = div_up(a.tiles_n, slices);
         const int rows  = div_up(div_up(a.block_rows, 4), bands);
@@ -145,7 +147,7 @@ __device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int slices, int& 
     }
     bx = l / a.tiles_n;
     by = l - bx * a.tiles_n;
-    if (!live) bx = a.block_rows;
+    if (!ONE && !live) bx = a.block_rows;
 }
 
 // ---------------------------------------------------------------------------
@@ -198,7 +200,7 @@ __global__ __launch_bounds__(256) void bsr_wave_kernel(BsrArgs a) {
     const int g    = lane >> 4;
     const int t    = lane & 15;
     int bx, by;
-    wave_tile_of(a, 1, bx, by);
+    wave_tile_of<true>(a, 1, bx, by);
     const int br   = bx * 4 + wave;
     const int n0   = by * NT;
     if (br >= a.block_rows) return;  // waves are independent: no barrier anywhere
@@ -360,7 +362,7 @@ __device__ u32x4 sbuf_load_u32x4_dev(__amdgpu_buffer_rsrc_t rsrc, int index, int
     return sbuf_load_u32x4(rsrc, index, offset, 0, 0);
 }
 
-template <int J, int D>
+template <int J, int D, bool ONE = false>
 __device__ __forceinline__ void bsr_record_body(const BsrArgs& a, int slices,
                                                 _Float16* __restrict__ s0,
                                                 _Float16* __restrict__ s1,
@@ -377,7 +379,7 @@ __device__ __forceinline__ void bsr_record_body(const BsrArgs& a, int slices,
     const int g    = lane >> 4;
     const int t    = lane & 15;
     int bx, by;
-    wave_tile_of(a, slices, bx, by);
+    wave_tile_of<ONE>(a, slices, bx, by);
     const int br   = bx * 4 + wave;
     const int n0   = by * NT;
     if (br >= a.block_rows) return;  // waves are independent: no barrier anywhere
@@ -543,7 +545,7 @@ __device__ __forceinline__ void bsr_record_body(const BsrArgs& a, int slices,
 // inlining, every slot access carries its own alias scope, which lets the
 // compiler's wait-count pass tell a read of slot d from the buffer-to-LDS
 // writes still in flight into the other slots.
-template <int J, int D>
+template <int J, int D, bool SLICES>
 __global__ __launch_bounds__(256) void bsr_record_kernel(BsrArgs a) {
     constexpr int TILE = 32 * 16 * J;
     static_assert(D == 2 || D == 4, "ring depth 2 or 4");
@@ -551,13 +553,13 @@ __global__ __launch_bounds__(256) void bsr_record_kernel(BsrArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 s_b1[4 * TILE];
     __shared__ __attribute__((aligned(16))) _Float16 s_b2[D == 4 ? 4 * TILE : 8];
     __shared__ __attribute__((aligned(16))) _Float16 s_b3[D == 4 ? 4 * TILE : 8];
-    int slices = a.slices;
-    if (slices > 1) {
+    if constexpr (SLICES) {
         RunSample sample;
         sample.load(a);
-        if (sample.in_runs()) slices = 1;
+        bsr_record_body<J, D>(a, sample.in_runs() ? 1 : a.slices, s_b0, s_b1, s_b2, s_b3);
+    } else {
+        bsr_record_body<J, D, true>(a, 1, s_b0, s_b1, s_b2, s_b3);
     }
-    bsr_record_body<J, D>(a, slices, s_b0, s_b1, s_b2, s_b3);
 }
 
 // ---------------------------------------------------------------------------
@@ -665,11 +667,8 @@ __device__ __forceinline__ bool bsr_panel_body(const BsrArgs& a, _Float16* __res
     const int wr   = wave / WC;
     const int wc   = wave % WC;
     int bx, by;
-    wave_tile_of(a, 1, bx, by);
-    const int br0 = bx * R;
-    // No tile: the whole workgroup leaves, before any barrier (or, to choose,
-    // has a panel of empty block-rows at hand).
-    if (!CHOOSE && br0 >= a.block_rows) return true;
+    wave_tile_of<!CHOOSE>(a, 1, bx, by);
+    const int br0 = bx * R;  // to choose, a workgroup without a tile has empty block-rows
     const int n0  = by * NT;
     auto stage = [&](int d) -> _Float16* { return d == 0 ? s0 : d == 1 ? s1 : d == 2 ? s2 : s3; };
 
@@ -1275,8 +1274,14 @@ hipError_t run_wave(BsrArgs args, hipStream_t stream, bool pointer_addressing) {
     args.wg_total = static_cast<int>(total);
     const unsigned tiles = slice_grid(args);
     if (!pointer_addressing && records_fit(args)) {
-        hipLaunchKernelGGL((bsr_record_kernel<J, D == 1 ? 2 : D>), dim3(tiles), dim3(256), 0,
-                           stream, args);
+        constexpr int DEPTH = D == 1 ? 2 : D;
+        if (args.slices > 1) {
+            hipLaunchKernelGGL((bsr_record_kernel<J, DEPTH, true>), dim3(tiles), dim3(256), 0,
+                               stream, args);
+        } else {
+            hipLaunchKernelGGL((bsr_record_kernel<J, DEPTH, false>), dim3(tiles), dim3(256), 0,
+                               stream, args);
+        }
         return hipGetLastError();
     }
     if (args.b_vec_ok) {
