@@ -598,13 +598,15 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
                     // on two paths would have to arrive before the paths join.
                     auto step = [&](int at0, auto refill) {
                         const bool ends = __ballot(row_len < at0 + U) != 0;
+                        // Pointer loads cannot read zeros for entries past a range.
+                        const bool past = !SBUF && __ballot(at0 + U > pb - pa) != 0;
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
                             if (__builtin_expect(ends, 0)) {
                                 if (at0 + u == row_len) flush(at0 + u);
                             }
                             VT& a_u = acc[u % kChains];
-                            if (SBUF || at0 + u < pb - pa) a_u = vv[u] * bv[u] + a_u;
+                            if (!past || at0 + u < pb - pa) a_u = vv[u] * bv[u] + a_u;
                             if constexpr (decltype(refill)::value) {
                                 __builtin_amdgcn_sched_barrier(0);  // into the registers just used
                                 vv[u] = entry_value(next[u]);
@@ -1371,13 +1373,18 @@ hipError_t dispatch_wide(int waves, const RowblockArgs& args, int grid, hipStrea
 // that are no whole number of lines keep 64 columns: every one touches a line
 // more (131072^2, 8 per row, N = 500: 414 us with 4 slices, 447 with 8; 65536^2, 32
 // per row, N = 96 99 us whole, 131 with 2; N = 192 226 with 2, 263 with 4).
-int auto_slices(int K, int N, double avg_row) {
+// wide: slices of at least 64 columns and none for the half of an L2.  For groups of
+// a number asked for, whose lanes narrower slices would leave idle (8192^2, 82 per
+// row, N = 256, one group: 50 us with two slices, 80 with four), and B past the
+// buffer's 2 GiB, which no slice brings near an L2 (65536 x 2.2 M, 24 per row, N = 256
+// 327 us with four, 361 with eight).
+int auto_slices(int K, int N, double avg_row, bool wide) {
     const long long b_bytes = static_cast<long long>(K) * N * 4;
     if (b_bytes <= (4LL << 20)) return 1;
-    const auto narrowest = [&](int slices) { return N % (32 * slices) == 0 ? 32 : 64; };
+    const auto narrowest = [&](int slices) { return !wide && N % (32 * slices) == 0 ? 32 : 64; };
     int s = 1;
     while (s < 8 && ((b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest(2 * s)) ||
-                     (b_bytes > (2LL << 20) * s && N / (2 * s) >= 64 && avg_row >= 16.0))) {
+                     (!wide && b_bytes > (2LL << 20) * s && N / (2 * s) >= 64 && avg_row >= 16.0))) {
         s *= 2;
     }
     return s;
@@ -1714,7 +1721,12 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     const double avg = A.nnz > 0 ? static_cast<double>(A.nnz) / M : 1.0;
     // Column slices (XCD-aware, see the kernel): 1, 2, 4 or 8.
     int slices = o.slices;
-    if (slices == 0) slices = role == CsrRole::Tiled ? 1 : auto_slices(A.num_cols, N, avg);
+    const bool sbuf = o.global_loads == 0 && b_fits_buffer(A.num_cols, N);
+    if (slices == 0) {
+        slices = role == CsrRole::Tiled
+                     ? 1
+                     : auto_slices(A.num_cols, N, avg, want_groups != 0 || !sbuf);
+    }
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     int slice_cols = ceil_div(N, slices);
     slice_cols = ceil_div(slice_cols, vec) * vec;
@@ -1727,7 +1739,6 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     // it: many small workgroups keep skewed rows balanced.  Rows known to be
     // even (max_row_hint): the whole-round grid of 4-wave workgroups.
     const int unroll = o.unroll == 8 ? 8 : 4;
-    const bool sbuf = o.global_loads == 0 && b_fits_buffer(A.num_cols, N);
 
     RowblockArgs args{};
     RowblockPart& part = args.part;
