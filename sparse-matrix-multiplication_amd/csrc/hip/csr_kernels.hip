@@ -1297,18 +1297,26 @@ long sliced_grid(long nblocks, int slices) {
 // Lane groups of a wave: with L = lanes of one row (slice) and p column passes
 // a group takes ceil(L / p) lanes; the pass count with the fewest passes per
 // entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
-void set_groups(RowblockArgs& a, int cols, int vec, int want) {
+// per_wave: entries of a wave.  More passes need 12 entries a group, 40 on merge-path
+// parts (power-law 2048^2, mean 64, N = 260 24.6 us in two passes, 29.1 in four; 8192^2,
+// mean 40 50 against 36), and those take no more groups than have 8: every part may
+// end in rows whose pieces the owner adds one by one (the first at N = 16 11.1 us
+// with eight waves' reductions, 14.2 with 64 groups of 4 entries).
+void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
     const int lanes = ceil_div(cols, vec);
     if (want == 1 || want == 2 || want == 4 || (want == 8 && vec == 4)) {
         a.groups      = want;
         a.group_lanes = kWave / want;
     } else {
+        const bool split = a.part.split_rows != nullptr;
+        const int most = split ? static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups))
+                               : kMaxGroups;
         int passes = ceil_div(lanes, kWave), best = passes;
-        const auto groups_of = [&](int p) {
-            return std::min(kMaxGroups, kWave / ceil_div(lanes, p));
-        };
+        const auto groups_of = [&](int p) { return std::min(most, kWave / ceil_div(lanes, p)); };
         for (int p = passes + 1; p <= 2 * passes; ++p) {
-            if (4 * p * groups_of(best) < 3 * best * groups_of(p)) best = p;
+            if (4 * p * groups_of(best) < 3 * best * groups_of(p) && per_wave >= (split ? 40 : 12) * groups_of(p)) {
+                best = p;
+            }
         }
         a.group_lanes = ceil_div(lanes, best);
         a.groups      = groups_of(best);
@@ -1748,7 +1756,16 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     args.N          = N;
     args.slices     = slices;
     args.slice_cols = slice_cols;
-    set_groups(args, slice_cols, vec, want_groups);
+    const long per_wave = split != nullptr    ? A.nnz / (4L * split->parts)
+                          : bounds != nullptr ? A.nnz / (8L * parts)
+                                              : std::min(160L, A.nnz / (slices == 1 ? 8L * 512 : 4L * 256));
+    if (split != nullptr) {
+        part.split_rows = split->rows;
+        part.carry      = split->carry;
+        part.nnz        = A.nnz;
+        part.nblocks    = split->parts;
+    }
+    set_groups(args, slice_cols, vec, want_groups, per_wave);
     // The whole-round grid is for few groups: it leaves more of them too few
     // row pieces each (65536^2, 40 per row, N = 256, eight slices of four groups:
     // 305 us with it, 260 without).
@@ -1757,15 +1774,10 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     const int waves = (o.waves == 2 || o.waves == 4 || o.waves == 8) ? o.waves
                       : even || slices > 1 || split != nullptr       ? 4
                                                                      : 8;
-    if (split != nullptr) {
-        part.split_rows = split->rows;
-        part.carry      = split->carry;
-        part.nnz        = A.nnz;
-        part.nblocks    = split->parts;
-    } else if (bounds != nullptr) {
+    if (bounds != nullptr) {
         args.bounds  = bounds;
         part.nblocks = parts;
-    } else {
+    } else if (split == nullptr) {
         int rpb = o.rows_per_block;
         if (rpb <= 0 && even) {
             rpb = round_rows_per_block(M, A.nnz, slices, waves);
@@ -1953,7 +1965,7 @@ Error launch_csr_khalf(const KHalfPlan& p, const float* B, float* C, hipStream_t
     args.M          = p.M;
     args.N          = N;
     args.slice_cols = N;
-    set_groups(args, N, 4, 0);
+    set_groups(args, N, 4, 0, std::min(args.part.nnz / p.parts[0], args.upper.nnz / p.parts[1]) / 4);
     const int grid   = 8 * ceil_div(std::max(p.parts[0], p.parts[1]), 4);
     hipError_t e = args.groups <= 2 ? dispatch_wide<true>(4, args, grid, stream)
                                     : run_rowblock<4, 4, 4, true, true>(args, grid, stream);
