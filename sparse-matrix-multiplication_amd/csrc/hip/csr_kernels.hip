@@ -327,7 +327,7 @@ __device__ __forceinline__ float entry_value(Entry e) {
     return __builtin_bit_cast(float, static_cast<uint32_t>(e >> 32));
 }
 
-template <int VEC, int WAVES, int U, bool SBUF, bool HALVES>
+template <int VEC, int WAVES, int U, bool SBUF, bool HALVES, bool FOLD>
 __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(RowblockArgs a) {
     using VT = typename Vec<VEC>::T;
     static_assert(kWCap % kWave == 0 && kMinWindow % U == 0, "whole steps per window");
@@ -543,7 +543,19 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
                 for (int i = 0; i < kChains; ++i) acc[i] = vzero<VEC>();
             };
             const auto sum = [&] { return (acc[0] + acc[1]) + (acc[2] + acc[3]); };
+            // v plus the pieces of local row r that groups from w on put aside, in two chains.
+            auto add_pieces = [&](VT v, int w, int r) {
+                const int at = place().glane;
+                VT odd = vzero<VEC>();
+                for (; w < NG && s_first[w] == r; w += 2) {
+                    v += s_part[w * lpg + at];
+                    if (w + 1 == NG || s_first[w + 1] != r) break;
+                    odd += s_part[(w + 1) * lpg + at];
+                }
+                return v + odd;
+            };
             clear();
+            VT folded = vzero<VEC>();  // FOLD: the row's sum over earlier windows
             if (wlen > 0) {
                 int  row  = first;
                 bool head = s_rp[row] < pa;  // row began in an earlier group
@@ -558,7 +570,11 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
                 int next_end = s_rp[row + 2 <= nr ? row + 2 : nr];
 
                 auto flush = [&](int at) {
-                    const VT done = sum();
+                    VT done = sum();
+                    if constexpr (FOLD) {
+                        done += folded;
+                        folded = vzero<VEC>();
+                    }
                     if (head) {
                         put_piece(row, done);
                         head = false;
@@ -623,9 +639,16 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
                         asm volatile("" : "+v"(at_kv));  // one address, the reads at constant offsets
                     }
                     step(win + q, std::false_type());
+                    if constexpr (FOLD) {  // chains no longer than a window's
+                        if (win + cap < wlen) {
+                            folded += sum();
+                            clear();
+                        }
+                    }
                 }
                 // The row being accumulated when the range ends.
                 acc[0] = sum();
+                if constexpr (FOLD) acc[0] += folded;
                 if (pa < pb) {
                     if (head) {
                         put_piece(row, acc[0]);
@@ -637,23 +660,14 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
                 }
             }
             __syncthreads();
-            const Place me = place();
+            const int gi_now = place().gi;
             if (owner_row >= 0) {
-                for (int w = me.gi + 1; w < NG; ++w) {
-                    if (s_first[w] != owner_row) break;
-                    acc[0] += s_part[w * lpg + me.glane];
-                }
-                store_row(m.C, w0 + owner_row, acc[0]);
+                store_row(m.C, w0 + owner_row, add_pieces(acc[0], gi_now + 1, owner_row));
             }
-            if (wg_head >= 0 && w0 == r_begin && me.gi == 0) {
+            if (wg_head >= 0 && w0 == r_begin && gi_now == 0) {
                 // The part's first row began in an earlier part: the groups that
                 // hold pieces of it (local row 0, leading groups) go to the carry.
-                VT piece = vzero<VEC>();
-                for (int w = 0; w < NG; ++w) {
-                    if (s_first[w] != 0) break;
-                    piece += s_part[w * lpg + me.glane];
-                }
-                store_row(m.carry, rb, piece);
+                store_row(m.carry, rb, add_pieces(vzero<VEC>(), 0, 0));
             }
             __syncthreads();  // s_part / s_first are rewritten by the next column pass
         }
@@ -1309,8 +1323,9 @@ void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
         a.group_lanes = kWave / want;
     } else {
         const bool split = a.part.split_rows != nullptr;
-        const int most = split ? static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups))
-                               : kMaxGroups;
+        const int most = split
+                             ? static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups))
+                             : kMaxGroups;
         int passes = ceil_div(lanes, kWave), best = passes;
         const auto groups_of = [&](int p) { return std::min(most, kWave / ceil_div(lanes, p)); };
         for (int p = passes + 1; p <= 2 * passes; ++p) {
@@ -1328,11 +1343,20 @@ void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
     while ((2 << a.window_log) * a.groups <= kWCap) ++a.window_log;
 }
 
-template <int VEC, int WAVES, int U, bool SBUF, bool HALVES = false>
+template <int VEC, int WAVES, int U, bool SBUF, bool HALVES = false, bool FOLD = false>
 hipError_t run_rowblock(const RowblockArgs& args, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((csr_rowblock<VEC, WAVES, U, SBUF, HALVES>), dim3(grid), dim3(WAVES * kWave), 0,
-                       stream, args);
+    hipLaunchKernelGGL((csr_rowblock<VEC, WAVES, U, SBUF, HALVES, FOLD>), dim3(grid),
+                       dim3(WAVES * kWave), 0, stream, args);
     return hipGetLastError();
+}
+
+// Merge-path ranges of eight groups and more fold their chains at every window's
+// end: csr_rowblock_wide's form had as many interleaved chains there, and four
+// over a whole range are up to 18% further from 64 bits (30000^2, 120 per row, N = 32
+// 0.86e-7 of the norm, 1.01e-7 and, folded, 0.78e-7; 34.5 -> 35 us).  Fewer groups and
+// shorter ranges need none.
+bool fold_windows(const RowblockArgs& a) {
+    return a.part.split_rows != nullptr && a.groups >= 8;
 }
 
 // Launch shapes: waves per workgroup (2, 4, 8) x entries in flight per group
@@ -1342,6 +1366,9 @@ template <int VEC>
 hipError_t dispatch_shape(int waves, int unroll, bool sbuf, const RowblockArgs& args, int grid,
                           hipStream_t stream) {
     if (!sbuf) return run_rowblock<VEC, 8, 4, false>(args, grid, stream);
+    if (waves == 4 && unroll == 4 && fold_windows(args)) {
+        return run_rowblock<VEC, 4, 4, true, false, true>(args, grid, stream);
+    }
     if (waves == 8) {
         return unroll == 8 ? run_rowblock<VEC, 8, 8, true>(args, grid, stream)
                            : run_rowblock<VEC, 8, 4, true>(args, grid, stream);
@@ -1765,6 +1792,7 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
         part.nnz        = A.nnz;
         part.nblocks    = split->parts;
     }
+    args.bounds = split == nullptr ? bounds : nullptr;
     set_groups(args, slice_cols, vec, want_groups, per_wave);
     // The whole-round grid is for few groups: it leaves more of them too few
     // row pieces each (65536^2, 40 per row, N = 256, eight slices of four groups:
@@ -1774,8 +1802,7 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     const int waves = (o.waves == 2 || o.waves == 4 || o.waves == 8) ? o.waves
                       : even || slices > 1 || split != nullptr       ? 4
                                                                      : 8;
-    if (bounds != nullptr) {
-        args.bounds  = bounds;
+    if (args.bounds != nullptr) {
         part.nblocks = parts;
     } else if (split == nullptr) {
         int rpb = o.rows_per_block;
@@ -1968,7 +1995,9 @@ Error launch_csr_khalf(const KHalfPlan& p, const float* B, float* C, hipStream_t
     set_groups(args, N, 4, 0, std::min(args.part.nnz / p.parts[0], args.upper.nnz / p.parts[1]) / 4);
     const int grid   = 8 * ceil_div(std::max(p.parts[0], p.parts[1]), 4);
     hipError_t e = args.groups <= 2 ? dispatch_wide<true>(4, args, grid, stream)
-                                    : run_rowblock<4, 4, 4, true, true>(args, grid, stream);
+                   : fold_windows(args)
+                       ? run_rowblock<4, 4, 4, true, true, true>(args, grid, stream)
+                       : run_rowblock<4, 4, 4, true, true>(args, grid, stream);
     if (e == hipSuccess) {
         const long long chunks = static_cast<long long>(p.M) * N / 4;
         hipLaunchKernelGGL(csr_khalf_fixup, dim3(static_cast<unsigned>((chunks + 255) / 256)),
