@@ -1313,7 +1313,7 @@ long sliced_grid(long nblocks, int slices) {
 // entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
 // per_wave: entries of a wave.  More passes need 12 entries a group, 40 on merge-path
 // parts (power-law 2048^2, mean 64, N = 260 24.6 us in two passes, 29.1 in four; 8192^2,
-// mean 40 50 against 36), and those take no more groups than have 8: every part may
+// mean 40 50 against 36), and those and explicit partitions take no more than have 8: every part may
 // end in rows whose pieces the owner adds one by one (the first at N = 16 11.1 us
 // with eight waves' reductions, 14.2 with 64 groups of 4 entries).
 void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
@@ -1323,7 +1323,7 @@ void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
         a.group_lanes = kWave / want;
     } else {
         const bool split = a.part.split_rows != nullptr;
-        const int most = split
+        const int most = split || a.bounds != nullptr
                              ? static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups))
                              : kMaxGroups;
         int passes = ceil_div(lanes, kWave), best = passes;
