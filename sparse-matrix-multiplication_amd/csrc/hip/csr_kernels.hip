@@ -1649,9 +1649,23 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
 // Column lanes: the fewest (a power of two, at most 64) that cover N; wider N in
 // column tiles of 256, a workgroup each.  Rows past a launch's threads (67 M at 64
 // lanes) go into further launches.
+// A whole wave takes each row at up to 8 columns where the rows are few and hold
+// 16 entries and more: the chip is nearly empty then, one row's chain is the whole
+// time, and the wave has its entries and 16 B rows in flight where a lane or two
+// waits for 8 entries and then for their B rows.  1000 rows of 451, N = 1 90 -> 20
+// us, N = 8 88 -> 24; 2048 rows of 63 14.6 -> 6.1 and 13.8 -> 8.1; 4096 rows of 157
+// 35.2 -> 13.9 and 30.8 -> 24.6.  Past that many rows the waves are what is waited
+// for: 8192 rows of 82, N = 3 17.2 -> 24.2, but N = 1 19.2 -> 13.4 still.  4096 rows
+// of 2, N = 8 3.0 -> 4.6.
+bool wave_a_row(int M, int nnz, int N) {
+    const double avg = static_cast<double>(nnz) / M;
+    return N <= 8 && avg >= 16.0 && M <= (N == 1 ? 8192 : avg >= 128.0 ? 5120 : 4096);
+}
+
 Error launch_in_order(const CSR& A, const float* B, float* C, int N, hipStream_t stream) {
     const int  vec    = pick_vec(N, 0);
-    const int  lc_log = pow2_log_at_least(ceil_div(N, vec));
+    const bool wave   = wave_a_row(A.num_rows, A.nnz, N);
+    const int  lc_log = wave ? 6 : pow2_log_at_least(ceil_div(N, vec));
     const int  per_wg = 4 * (kWave >> lc_log);
     const long most   = kMaxThreads / 256 * per_wg;
     for (long first = 0; first < A.num_rows; first += most) {
@@ -1663,8 +1677,10 @@ Error launch_in_order(const CSR& A, const float* B, float* C, int N, hipStream_t
                                C + static_cast<size_t>(first) * N);
             return from_hip(hipGetLastError(), "csr in-order launch");
         };
-        const Error e = vec == 1      ? run(csr_rows_in_order<1, Hand::Direct>)
-                        : vec == 2    ? run(csr_rows_in_order<2, Hand::Direct>)
+        const Error e = vec == 1      ? run(wave ? csr_rows_in_order<1, Hand::Readlane>
+                                                 : csr_rows_in_order<1, Hand::Direct>)
+                        : vec == 2    ? run(wave ? csr_rows_in_order<2, Hand::Readlane>
+                                                 : csr_rows_in_order<2, Hand::Direct>)
                         : lc_log == 6 ? run(csr_rows_in_order<4, Hand::Readlane>)
                         : lc_log >= 3 ? run(csr_rows_in_order<4, Hand::Shuffle>)
                                       : run(csr_rows_in_order<4, Hand::Direct>);

@@ -137,6 +137,28 @@ def test_sequential_roles_are_the_reference_chain_bit_for_bit(S, O, torch, edge_
         assert np.array_equal(C.view(np.uint32), ref.view(np.uint32)), name
 
 
+@pytest.mark.parametrize("M", [13, 4096, 4097])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 7, 8, 9])
+def test_sequential_roles_few_long_rows(S, O, torch, M, N):
+    # A wave a row for few rows of 16 entries and more at up to 8 columns, lanes by
+    # the width otherwise (4097 rows stay with the wave at N = 1): the same chain.
+    # Rows end at and around the steps of 16 and the 64 entries a wave holds; some
+    # are empty, and an infinity in B reaches only the rows that have its entry.
+    K = 900
+    rng = np.random.default_rng(41)
+    lens = np.resize(np.array([0, 1, 15, 16, 17, 63, 64, 65, 129, 700, 2, 48, 0]), M)
+    col = np.concatenate([np.sort(rng.choice(K, n, replace=False)) for n in lens]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    A = S.HostCSR(M, K, rp, col, rng.uniform(-1, 1, col.size).astype(np.float32))
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    B[K // 2] = np.inf
+    ref = O.csr_spmm_f32_fma(A.row_ptr, A.col_idx, A.values, B)
+    for kernel in ("baseline", "memopt", "memopt_v2"):
+        say(f"csr {kernel} few long rows M={M} N={N}")
+        C = _run(S, torch, kernel, A, B)
+        assert np.array_equal(C.view(np.uint32), ref.view(np.uint32)), kernel
+
+
 @pytest.mark.parametrize("cfg", ["c1", "c2"])
 def test_row_groups_one_entry_lane_is_the_reference_chain(S, O, torch, config_refs, cfg):
     # The tiled roles' fast forms associate a row's sum differently from the
