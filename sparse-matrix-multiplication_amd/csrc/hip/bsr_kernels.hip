@@ -635,6 +635,39 @@ __device__ __forceinline__ uint64_t below(int p) {  // bits 0 .. p-1, p in [0, 6
     return (1ull << p) - 1ull;
 }
 
+// Block-rows br0 .. br0+rows-1 of `tiles` 16-column tiles from n0, by one wave and
+// block by block straight from memory: what a panel's wave does with sums that are
+// not finite.  The order of the sums is the panel's.
+__device__ void bsr_tiles_apart(const BsrArgs& a, int br0, int rows, int n0, int tiles, int lane) {
+    const int g = lane >> 4, t = lane & 15;
+    for (int br = br0; br < min(br0 + rows, a.block_rows); ++br) {
+        for (int j = 0; j < tiles; ++j) {
+            const int col = n0 + 16 * j + t;
+            f32x4 acc = f32x4(0.0f);
+            for (int e = a.row_ptr[br]; e < a.row_ptr[br + 1]; ++e) {
+                const int  bc = a.col_idx[e];
+                const bool in = static_cast<unsigned>(bc) < static_cast<unsigned>(a.block_cols);
+                f16x4 b;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int  k  = bc * 16 + 4 * g + i;
+                    const bool ok = in && k < a.K && col < a.N;
+                    b[i] = ok ? a.B[static_cast<size_t>(k) * a.N + col] : static_cast<_Float16>(0.0f);
+                }
+                const f16x4 av = *reinterpret_cast<const f16x4*>(
+                    a.vals + static_cast<size_t>(e) * 256 + t * 16 + 4 * g);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16f16(av, b, acc, 0, 0, 0);
+            }
+            if (col >= a.N) continue;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int row = br * 16 + 4 * g + k;
+                if (row < a.M) store_c(a.C + static_cast<size_t>(row) * a.N + col, acc[k]);
+            }
+        }
+    }
+}
+
 // CHOOSE: returns false, with nothing done, where A's blocks lie in no runs.
 // The sample's loads go out before the panel's own and wait with them.
 template <int R, int J, int WR, int D, bool CHOOSE = false>
@@ -1015,6 +1048,22 @@ __device__ __forceinline__ bool bsr_panel_body(const BsrArgs& a, _Float16* __res
                 if (row < a.M) store_c(a.C + static_cast<size_t>(row) * a.N + col, acc[i][j][k]);
             }
         }
+    }
+    // A block-row's pair is multiplied with the B rows of both its slots, those
+    // of a block that it has not by an A of zeros: an infinity or a NaN there, of
+    // another block-row's, would be in its sums.  Looked for behind the stores,
+    // which the lanes then write again.
+    f32x4 z = f32x4(0.0f);
+#pragma unroll
+    for (int i = 0; i < TR; ++i) {
+#pragma unroll
+        for (int j = 0; j < TC; ++j) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) z[k] = __builtin_fmaf(acc[i][j][k], 0.0f, z[k]);
+        }
+    }
+    if (__builtin_expect(__any((z[0] + z[1]) + (z[2] + z[3]) != 0.0f), 0)) {
+        bsr_tiles_apart(a, br0 + wr * TR, TR, n0 + wc * TC * 16, TC, lane);
     }
     return true;
 }

@@ -510,3 +510,48 @@ def test_wmma_strewn_or_runs(S, torch, pattern, M, K, N, lo, hi):
     S.spmm_wmma(S.DeviceBSR(hb), B, C)
     torch.cuda.synchronize()
     check_csr(C.cpu().numpy(), C64.cpu().numpy(), absC.cpu().numpy(), tol=1e-5)
+
+
+@pytest.mark.parametrize("M,K,N,lo,hi,opts", [
+    (500, 1293, 100, 3, 9, {}),              # chunks at any element, odd and even lists
+    (500, 1293, 33, 1, 4, {}),               # the same, one tile
+    (500, 1293, 64, 3, 9, {"addressing": 1}),  # whole chunks by pointer
+    (500, 1293, 128, 3, 9, {}),              # records
+    (5003, 9001, 328, 26, 62, {}),           # panel or pairs of waves
+    (8501, 6007, 512, 26, 62, {}),           # panel or single blocks, in slices
+    (500, 1293, 128, 20, 40, {"row_group": 4}),
+    (500, 1293, 136, 20, 40, {"row_group": 8, "tiles": 8}),
+])
+@pytest.mark.parametrize("pattern", ["strewn", "runs"])
+def test_wmma_nan_in_b(S, torch, M, K, N, lo, hi, opts, pattern):
+    # A NaN row of B reaches the rows whose block-row has its block-column and no
+    # others, which keep their bits: the clamped addresses that absent blocks
+    # read (row 0), the chunk that runs over into the next row (the first row of
+    # a block-column) and the shared panel's other block-rows add nothing.
+    rng = np.random.default_rng(M + N + hi)
+    br, bc = -(-M // 16), -(-K // 16)
+    count = lo + np.arange(br) % (hi - lo + 1)
+    row_ptr = np.concatenate([[0], count.cumsum()]).astype(np.int32)
+    cols = np.concatenate([np.arange(n) + (r * 3) % (bc - n + 1) if pattern == "runs"
+                           else np.sort(rng.choice(bc, n, replace=False))
+                           for r, n in enumerate(count)]).astype(np.int32)
+    vals = rng.integers(-99, 99, (cols.size, 16, 16)).astype(np.float16)
+    rows = np.repeat(np.arange(br), count)
+    vals[rows[:, None] * 16 + np.arange(16) >= M] = 0
+    vals.transpose(0, 2, 1)[cols[:, None] * 16 + np.arange(16) >= K] = 0
+    dA = S.DeviceBSR(S.HostBSR(M, K, br, bc, int((vals != 0).sum()), row_ptr, cols,
+                               vals.reshape(-1).view(np.uint16)))
+    B = torch.from_numpy(rng.uniform(-1, 1, (K, N)).astype(np.float16)).cuda()
+    bad = np.array([0, 16 * (bc // 2), K - 1])
+    B[bad] = 0
+    say(f"wmma NaN in B {pattern} M={M} K={K} N={N} {opts}")
+    o = S.BsrOptsT(**opts)
+    clean = torch.empty((M, N), device="cuda")
+    S.spmm_wmma_opts(dA, B, o, clean)
+    B[bad] = float("nan")
+    C = torch.empty((M, N), device="cuda")
+    S.spmm_wmma_opts(dA, B, o, C)
+    hit = torch.from_numpy(np.repeat(np.isin(np.arange(br), rows[np.isin(cols, bad // 16)]), 16)[:M])
+    assert hit.any() and not hit.all()
+    assert torch.isnan(C[hit.cuda()]).all()
+    assert torch.equal(C[~hit.cuda()].view(torch.int32), clean[~hit.cuda()].view(torch.int32))
