@@ -1033,7 +1033,6 @@ __device__ __forceinline__ bool bsr_panel_body(const BsrArgs& a, _Float16* __res
     }
 
 
-
     // D layout: lane holds rows 4*g + i, column t of each 16-column tile.
 #pragma unroll
     for (int i = 0; i < TR; ++i) {

@@ -411,9 +411,11 @@ def test_wmma_any_width_and_alignment(S, O, torch, N, shift):
     # 16-byte chunks of B rows that start at any fp16 element, the last chunk
     # of a row running into the next row and, at B's end, taken from before it.
     # B and C start `shift` elements past an aligned address inside buffers
-    # whose other elements are NaN: a read outside B would show in C (every
-    # column of the last block-column's rows is multiplied), a write outside C
-    # would change a NaN.  K = 1 with N < 8 is smaller than one chunk.
+    # whose other elements are NaN: a wrong shift of the last chunk puts a NaN or
+    # a neighbour's product into C, a write outside C changes a NaN.  A read
+    # outside B whose elements are then dropped does not show here; that no
+    # chunk makes one is checked where the kernel is compiled (chunks_inside).
+    # K = 1 with N < 8 is smaller than one chunk.
     for M, K, dens in ((70, 150, 0.2), (33, 47, 1.0), (40, 1, 1.0)):
         A = S.generate_uniform_random_csr(M, K, dens, 7 + N)
         A.values = S.round_to_fp16(A.values)
@@ -438,9 +440,10 @@ def test_wmma_any_width_and_alignment(S, O, torch, N, shift):
 @pytest.mark.parametrize("M,K,N", [(1007, 1600, 320), (530, 1293, 648), (2100, 8200, 512),
                                    (100, 5300, 1024)])
 def test_wmma_wide_b(S, O, torch, pattern, M, K, N):
-    # Wide B and 24 - 64 blocks per block-row: blocks in runs take the shared
-    # panel, others the waves, over column slices where B is over 5 MiB; row
-    # groups and column tiles that the XCDs' shares do not divide.
+    # Wide B and 24 - 64 blocks per block-row, row groups and column tiles that
+    # the XCDs' shares do not divide: 2100 rows and N = 512 are more than 256
+    # workgroups, where the launch looks and takes the panel for runs and the
+    # waves for others, over column slices; the rest take the record kernel.
     rng = np.random.default_rng(M + N)
     br, bc = -(-M // 16), -(-K // 16)
     row_ptr, cols = [0], []

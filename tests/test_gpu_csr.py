@@ -699,3 +699,41 @@ def test_row_groups_column_slices(S, O, torch, N):
     S.spmm_tiled_v3_opts(dA, dB, S.EngineOptsT(row_groups=1), C)
     torch.cuda.synchronize()
     check_csr(C.cpu().numpy(), C64, absC)
+
+
+@pytest.mark.parametrize("N", [1, 4, 20, 64, 100, 128, 200, 256, 300])
+def test_nan_in_b(S, torch, N):
+    # A NaN row of B reaches the rows with an entry in its column and no others,
+    # which keep their bits: the entries that fill up a step or a window, the lanes
+    # past a row's end and neighbouring rows of a group add nothing.
+    M, K = 1301, 701
+    rng = np.random.default_rng(N)
+    lens = np.resize(np.array([0, 1, 2, 3, 5, 8, 9, 31, 33, 64, 65, 0, 130, 4, 7, 350, 1, 0]), M)
+    col = np.concatenate([np.sort(rng.choice(K, n, replace=False)) for n in lens]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    A = S.HostCSR(M, K, rp, col, rng.uniform(-1, 1, col.size).astype(np.float32))
+    bad = np.array([0, K // 2, K - 1])
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    B[bad] = 0
+    dA, clean = S.DeviceCSR(A), torch.from_numpy(B).cuda()
+    dirty = clean.clone()
+    dirty[bad] = float("nan")
+    E = S.EngineOptsT
+    bounds = torch.from_numpy(S.nnz_balanced_bounds(A, 37)).cuda()
+    parts = torch.from_numpy(S.nnz_split_rows(A, 37)).cuda()
+    runs = {k: lambda b, k=k: S.spmm_csr(k, dA, b) for k in KERNELS if k != "tiled_v2" or N % 128 == 0}
+    for o in (E(max_row_hint=350), E(vec=1, groups=2), E(vec=2, unroll=8), E(global_loads=1), E(slices=2),
+              E(vec=4, groups=4, unroll=2), E(row_groups=1), E(row_groups=2), E(row_groups=3),
+              E(row_groups=2, entry_lanes=8, slices=2)):
+        runs[tuple((n, getattr(o, n)) for n, _ in E._fields_ if getattr(o, n))] = (
+            lambda b, o=o: S.spmm_tiled_v3_opts(dA, b, o))
+    runs["split"] = lambda b: S.spmm_tiled_v3_split(dA, parts, b)
+    runs["bounds"] = lambda b: S.spmm_tiled_v3_partitioned(dA, bounds, b)
+    hit = np.zeros(M, bool)
+    hit[np.repeat(np.arange(M), lens)[np.isin(col, bad)]] = True
+    hit = torch.from_numpy(hit).cuda()
+    for name, run in runs.items():
+        say(f"csr NaN in B N={N} {name}")
+        want, got = run(clean), run(dirty)
+        assert torch.isnan(got[hit]).all(), name
+        assert torch.equal(got[~hit].view(torch.int32), want[~hit].view(torch.int32)), name
