@@ -85,9 +85,13 @@ typedef struct spmm_hybrid_plan_t {
 typedef struct spmm_engine_opts_t {
     int vec;            /* floats per lane per B load: 1, 2, 4 */
     int waves;          /* waves per workgroup: 2, 4, 8 */
-    int unroll;         /* B row segments per lane per step (two steps in flight): 4, 8 */
+    int unroll;         /* B row segments in flight per lane: 4, 8 */
     int rows_per_block; /* implicit partition granularity */
-    int groups;         /* lane groups per wave, entries interleaved: 1, 2, 4 */
+    int groups;         /* lane groups per wave, a contiguous range of entries each:
+                           1, 2, 4 or (vec 4) 8; 0: as many as the columns of a
+                           pass leave lanes for.  Automatic launches of one or
+                           two groups on even rows or merge-path parts interleave
+                           the groups' entries instead */
     int slices;         /* XCD-tied column slices of B and C: 1, 2, 4, 8 */
     int global_loads;   /* 1: 64-bit address loads of B instead of buffer loads
                            (automatic when B exceeds 2 GiB or N > 4095) */
@@ -118,8 +122,9 @@ typedef struct spmm_engine_opts_t {
  * reference: exposes the kernels' variants for measurement sweeps.  Default:
  * the shared-panel kernel on wide B with long block-rows (N >= 256, 24 - 64
  * blocks per block-row on average, K <= 131072), else the wave kernel.  From one
- * block in 24 on the wave kernel for N < 320, and for wider B one launch that
- * takes the panel where A's blocks lie in runs and waves where they do not. */
+ * block in 24 on the wave kernel up to 256 panel workgroups (4 block-rows x 64
+ * columns each), and beyond one launch that takes the panel where A's blocks lie
+ * in runs and waves where they do not. */
 typedef struct spmm_bsr_opts_t {
     int row_group;  /* 0: automatic; 1: wave kernel (one wave per block-row);
                        4, 8: shared-panel kernel with that many block-rows per

@@ -159,8 +159,8 @@ __device__ __forceinline__ void wave_tile_of(const BsrArgs& a, int slices, int& 
 // col_idx -> (A, B) -> MFMA.  Latency and the B re-reads of every block-row
 // bound it.  Rows of B may start at any element: 16-byte chunks at any N and
 // alignment (MI355X against one load per element, which bound those widths
-// before: 5003 x 6997 blocks at 15%, N = 100 66.2 -> 15.1 us; 8192^2 at 12.5%, N =
-// 500 228 -> 46 us).
+// before: 5003 x 6997 blocks at 15%, N = 100 65.4 -> 15.6 us, one call from Python
+// 66.8 -> 17.6; 8192^2 at 12.5%, N = 500 226 -> 48 us).
 //   - The block-row's block-columns come in with one vector load (lane i
 //     holds col_idx[first + i], 64 per chunk) and are broadcast with
 //     v_readlane, so pairs need no further index loads.

@@ -3,6 +3,8 @@
 //   csr_rows_in_order  role of spmm_baseline and spmm_memopt/_v2
 //                      (spmm_baseline.cu:11-25, spmm_memopt.cu:11-38)
 //   csr_rowblock       role of spmm_tiled* (spmm_tiled_v3.cu:21-104), the engine
+//   csr_rowblock_wide  the engine on wide B and balanced partitions
+//   csr_row_groups     the engine's role on narrow B and short rows
 //
 // All accumulate in fp32 with fused multiply-adds.  C is fully written
 // (rows without nonzeros get zeros), so callers never clear it.
@@ -107,11 +109,10 @@ __device__ __forceinline__ typename Vec<VEC>::T vzero() {
 // TB/s).  Measured on MI355X against the form before it, in which the groups of
 // a wave took alternate entries of one range, in whole steps of U * G entries,
 // and reduced at every row end (csr_rowblock_wide is that form): 20011 x 17001,
-// 40 per row, N = 77 30.8 -> 23.7 us; 65536^2, 32 per row, N = 256 250 -> 211 us
+// 40 per row, N = 77 30.8 -> 22.6 us; 65536^2, 32 per row, N = 256 243 -> 209 us
 // with eight slices (298 in the old form, whose steps of 32 entries each held a
 // row end); power-law 65536^2, N = 32 over B-row halves 67 -> 35 us; 8192^2
-// power-law, N = 256 49.6 -> 29.1 us; 1.25x over 300 uniform and power-law
-// inputs.
+// power-law, 74 per row, N = 256 63 -> 40 us.
 //
 // Rows of the workgroup without nonzeros are zero-filled up front.  Row
 // pointers are staged in LDS in windows of kRpCap rows.
@@ -158,8 +159,9 @@ struct RowblockArgs {
 
 // Has every argument loaded before the first branch on one of them.  Left to
 // itself the compiler loads each group of arguments where it is first needed,
-// and every group costs a small launch one more wait on the scalar cache
-// (MI355X, 2048^2, 40 per row, N = 256: 6.84 against 6.63 us).
+// and every group costs a launch one more wait on the scalar cache (MI355X,
+// over 60 launches of 4 to 100 us 0.1 - 0.4 us; 2048^2, 40 per row, N = 256: 6.84
+// against 6.63 us).  The eight scalar registers that this spills cost less.
 __device__ __forceinline__ void load_args(const RowblockArgs& a, const RowblockPart& m) {
     asm volatile("" ::"s"(m.row_ptr), "s"(m.col_idx), "s"(m.vals), "s"(m.B), "s"(m.C),
                  "s"(m.split_rows), "s"(m.carry), "s"(m.nnz), "s"(m.K), "s"(m.nblocks),
@@ -232,10 +234,11 @@ __device__ __forceinline__ typename Vec<VEC>::T fma_vec(float v, typename Vec<VE
 // hands them out by readlane (L = 64: one row per wave, so the B row's address
 // is scalar) or shuffle; groups of under eight lanes load them directly.
 // Latency bounds it: U x resident waves loads in flight.  Measured on MI355X
-// against one wave per row with 4-byte lanes and one entry at a time: 4096^2, 41
-// per row, N = 256 64.9 -> 10.4 us (2.6 -> 16.5 TB/s of gathered rows), N = 128 22.5 ->
-// 6.8 us; 65536^2, 16 per row, N = 1 44.5 -> 8.3 us; and against one lane per output
-// (spmm_baseline before) 24.5 -> 10.4, 14.6 -> 6.8 and 39.0 -> 8.3 us.
+// (launches back to back; one call from Python 69 -> 11.7) against one wave per row
+// with 4-byte lanes and one entry at a time: 4096^2, 41 per row, N = 256 64.1 -> 10.4
+// us (2.7 -> 16.4 TB/s of gathered rows), N = 128 20.8 -> 6.7 us; 65536^2, 16 per row,
+// N = 1 45.0 -> 8.2 us; and against one lane per output (spmm_baseline before) 25.8 ->
+// 10.4, 13.9 -> 6.7 and 38.9 -> 8.2 us.
 // ---------------------------------------------------------------------------
 enum class Hand { Direct, Shuffle, Readlane };
 
@@ -685,9 +688,9 @@ __global__ __launch_bounds__(WAVES * 64, U == 8 ? 4 : 5) void csr_rowblock(Rowbl
 // per entry and starts half as many row pieces; csr_rowblock's groups wait for
 // nobody and win from three groups on and on uneven rows.  MI355X, this form
 // against csr_rowblock: 16384^2 power-law over B-row halves, N = 128 61.3 against
-// 62.7 us; 8192^2, 100 per row, N = 256 36.6 against 37.6; 2048^2, 250 per row,
-// N = 256 18.9 against 19.9; merge-path 8192^2 power-law, N = 32 (eight groups)
-// 19.0 against 14.2.
+// 62.7 us; 8192^2, 100 per row, N = 256 36.2 against 36.3, N = 128 19.6 against 20.3;
+// 2048^2, 235 per row, N = 256 19.1 against 19.9; merge-path 8192^2 power-law, N = 32
+// (eight groups) 19.0 against 14.2.
 // ---------------------------------------------------------------------------
 // Sum of the G groups' tiles, returned to every lane.
 template <int G>
@@ -1057,7 +1060,7 @@ __global__ __launch_bounds__(256) void csr_khalf_fixup(float* __restrict__ C,
 // with xor shuffles (fixed order) and entry lane 0 stores the row.
 //
 // For N of a few columns the row-block engine leaves most lanes idle (its
-// groups cover columns, at most 8 per wave) and pays its per-step row tests on
+// groups cover columns, at most 16 per wave) and pays its per-step row tests on
 // every entry; here a wave gathers 64 / LC entries per load instruction.
 // Measured on MI355X: 1.5 - 4x faster than the engine for N <= 32 on uniform
 // rows of 1 .. 300 entries, up to 2x at N = 64, and for N = 128 / 256 on rows
@@ -1564,8 +1567,9 @@ bool more_entry_lanes(int M, int K, int N, long long nnz, int max_row, int lc_lo
 // Shape of the sub-wave row groups, measured on MI355X over uniform rows of
 // 1 .. 300 entries, M = 2048 .. 65536 and N = 1 .. 256:
 //  - column lanes cover N in one pass (up to 64 lanes), except that 32 or 64
-//    column lanes drop to 16 (two or four passes) while the matrix would
-//    still give >= 16384 waves (e.g. M = 32768, N = 128: 96 -> 89 us);
+//    column lanes drop to 16 (two or four passes) where N is whole 128-byte
+//    lines and the matrix still gives >= 16384 waves (M = 32768, N = 128: 96 -> 89
+//    us; at other widths every pass would touch a line more);
 //  - entry lanes ~1.5 * sqrt(average row) as a power of two, but no more than
 //    keep the grid near 8192 waves (32 per CU): beyond that, more rows per wave
 //    beat more lanes per row -- except on the rows of more_entry_lanes;
@@ -1738,10 +1742,12 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     // row-length knowledge: 1.6 - 3.4x faster on uniform rows at N <= 8 and
     // 2.5 - 3.6x on power-law rows of up to 4096 entries; at N = 12 - 16 over
     // 32 uniform and power-law inputs (M 2048 .. 65536) 2.0x on average, never
-    // slower (1.18x at worst).  Up to eight lanes (N <= 32) they win 1.07 -
-    // 1.75x on the inputs of up to 2.5 M nonzeros but lose 0.79 - 0.97x on
-    // power-law inputs of 4.6 M nonzeros and more, so five to eight lanes take
-    // them only up to 4 M nonzeros.  Any explicit engine option keeps the
+    // slower (1.18x at worst).  At five to eight lanes (N <= 32) they win 1.07 -
+    // 1.75x on the inputs of up to 2.5 M nonzeros.  Past 4 M the engine stays: of
+    // larger inputs the row groups take some in less (20000 rows of 298, N = 32 36
+    // against 60 us; power-law 30000 of 147 51 against 64), others in more (65536 of
+    // 80, N = 20 62 against 60; 300000 of 16 97 against 95; power-law 131072 of 39
+    // 96 against 92), and no rule on sizes parts them yet.  Any explicit engine option keeps the
     // engine, and so does a longest-row hint: a caller that knows its rows
     // (spmm_hybrid_run) chooses the form itself.
     const bool engine_defaults = o.vec == 0 && o.waves == 0 && o.unroll == 0 &&
@@ -1785,7 +1791,8 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     // workgroup without column slices (a workgroup's nonzeros are split over
     // its waves, so a long row is shared by eight: power-law 2048^2, N = 128 9.5
     // us with 8, 12.1 with 4), 4 with them (more workgroups per row block) and
-    // on merge-path parts; 4 rows in flight per group; about 160 nonzeros per
+    // on merge-path parts, except csr_rowblock_wide's without slices (8, see
+    // wg_waves); 4 rows in flight per group; about 160 nonzeros per
     // wave and at least 512 row blocks (256 with slices) when the matrix allows
     // it: many small workgroups keep skewed rows balanced.  Rows known to be
     // even (max_row_hint): the whole-round grid of 4-wave workgroups.

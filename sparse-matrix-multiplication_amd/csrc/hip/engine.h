@@ -39,7 +39,7 @@ enum class CsrRole : int {
 struct EngineOpts {
     int vec            = 0;  // floats per lane per B load: 1, 2 or 4
     int waves          = 0;  // waves per workgroup: 2, 4 or 8
-    int unroll         = 0;  // B rows in flight per group: 4 or 8
+    int unroll         = 0;  // B row segments in flight per lane: 4 or 8
     int rows_per_block = 0;  // implicit partition: rows per workgroup
     int groups         = 0;  // lane groups per wave: 1, 2, 4 or (vec 4) 8; 0: as many as fit
     int slices         = 0;  // XCD-tied column slices of B and C: 1, 2, 4 or 8
@@ -87,7 +87,8 @@ Error launch_shader_clock_trace(unsigned long long* d_out, int samples, int inte
 
 // Tuning of the BSR matrix-core kernels.  All zero selects the default: the
 // shared-panel kernel on wide B with long structured block-rows (N >= 256, 24
-// - 64 blocks per block-row), else the wave kernel, with shapes from N.
+// - 64 blocks per block-row; from one block in 24 on a launch that looks for runs, or
+// up to 256 panel workgroups the waves), else the wave kernel, with shapes from N.
 struct BsrOpts {
     int row_group  = 0;  // 0: automatic; 1: wave kernel; 4, 8: panel kernel with that many
                          // block-rows per workgroup sharing staged B tiles
