@@ -1314,7 +1314,9 @@ long sliced_grid(long nblocks, int slices) {
 // Lane groups of a wave: with L = lanes of one row (slice) and p column passes
 // a group takes ceil(L / p) lanes; the pass count with the fewest passes per
 // entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
-// per_wave: entries of a wave.  More passes need 12 entries a group, 40 on merge-path
+// per_wave: entries of a wave.  More passes need 18 entries a group (1050 rows of 200,
+// N = 160 15.2 us in two passes of 51 entries, 12.2 in one; 2100 of 100, N = 320 25.2
+// and 23.4; 4096 of 60, 60 entries, 11.0 and 11.7), 40 on merge-path
 // parts (power-law 2048^2, mean 64, N = 260 24.6 us in two passes, 29.1 in four; 8192^2,
 // mean 40 50 against 36), and those and explicit partitions take no more than have 8: every part may
 // end in rows whose pieces the owner adds one by one (the first at N = 16 11.1 us
@@ -1332,7 +1334,7 @@ void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
         int passes = ceil_div(lanes, kWave), best = passes;
         const auto groups_of = [&](int p) { return std::min(most, kWave / ceil_div(lanes, p)); };
         for (int p = passes + 1; p <= 2 * passes; ++p) {
-            if (4 * p * groups_of(best) < 3 * best * groups_of(p) && per_wave >= (split ? 40 : 12) * groups_of(p)) {
+            if (4 * p * groups_of(best) < 3 * best * groups_of(p) && per_wave >= (split ? 40 : 18) * groups_of(p)) {
                 best = p;
             }
         }
