@@ -686,6 +686,44 @@ def test_row_groups_rounding(S, O, torch):
     assert rel <= bound, (rel, bound)
 
 
+@pytest.mark.parametrize("M,per,N", [(1050, 60, 160), (2100, 100, 320), (525, 9, 77), (4200, 41, 256),
+                                     (7000, 12, 200), (9000, 30, 160), (20000, 20, 160), (4000, 30, 512)])
+@pytest.mark.parametrize("pattern", ["even", "uneven"])
+def test_engine_grids_and_slices(S, torch, M, per, N, pattern):
+    # Row blocks just over a round of the chip, one and two passes per row, and the
+    # slices that depend on whether the rows are even: with the longest row as a
+    # hint and without, and as merge-path parts.
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    lens = torch.randint(per // 2, per + per // 2 + 1, (M,), generator=g, device="cuda")
+    if pattern == "uneven":
+        lens[::97] = min(20 * per, M)
+        lens[5::11] = 0
+    rp = torch.zeros(M + 1, dtype=torch.int32, device="cuda")
+    rp[1:] = lens.cumsum(0)
+    nnz = int(rp[-1])
+    col = torch.randint(0, M, (nnz,), generator=g, device="cuda", dtype=torch.int32)
+    val = torch.rand(nnz, generator=g, device="cuda") * 2 - 1
+    B = torch.rand((M, N), generator=g, device="cuda") * 2 - 1
+    rows = torch.repeat_interleave(torch.arange(M, device="cuda"), lens)
+    C64 = torch.zeros((M, N), dtype=torch.float64, device="cuda")
+    absC = torch.zeros_like(C64)
+    for i in range(0, nnz, 1 << 17):
+        p = val[i:i + (1 << 17), None].double() * B[col[i:i + (1 << 17)].long()].double()
+        C64.index_add_(0, rows[i:i + (1 << 17)], p)
+        absC.index_add_(0, rows[i:i + (1 << 17)], p.abs())
+    A = S.HostCSR(M, M, rp.cpu().numpy(), col.cpu().numpy(), val.cpu().numpy())
+    dA, parts = S.DeviceCSR(A), torch.from_numpy(S.nnz_split_rows(A, min(512, nnz))).cuda()
+    E = S.EngineOptsT
+    for name, run in (("plain", lambda C: S.spmm_csr("tiled_v3", dA, B, C)),
+                      ("hint", lambda C: S.spmm_tiled_v3_opts(dA, B, E(max_row_hint=int(lens.max())), C)),
+                      ("split", lambda C: S.spmm_tiled_v3_split(dA, parts, B, C))):
+        say(f"csr engine grid {pattern} {name} M={M} per={per} N={N}")
+        C = torch.full((M, N), float("nan"), device="cuda")
+        run(C)
+        torch.cuda.synchronize()
+        check_csr(C.cpu().numpy(), C64.cpu().numpy(), absC.cpu().numpy())
+
+
 @pytest.mark.parametrize("N", [100, 130, 198, 250, 499, 512])
 def test_row_groups_column_slices(S, O, torch, N):
     # B past an L2 under rows of up to 24: whole, or in two to eight slices whose
