@@ -1402,6 +1402,13 @@ hipError_t dispatch_wide(int waves, const RowblockArgs& args, int grid, hipStrea
                             : run(csr_rowblock_wide<2, 4, HALVES>);
 }
 
+// Rows whose lengths stay within twice the average (plus a constant for
+// short rows): uniform random rows qualify, power-law rows do not.
+bool rows_even(int M, long long nnz, int max_row) {
+    return max_row > 0 && M > 0 &&
+           max_row <= 2.0 * static_cast<double>(nnz) / M + 32.0;
+}
+
 // Column slices for a K x N fp32 B: the fewest (a power of two, at most 8) that
 // bring one XCD's share of B down to its 4 MiB L2, each at least 32 columns
 // wide (one 128-byte line of a B row); on rows of 16 entries and more, while
@@ -1418,28 +1425,40 @@ hipError_t dispatch_wide(int waves, const RowblockArgs& args, int grid, hipStrea
 // row, N = 256, one group: 50 us with two slices, 80 with four), and B past the
 // buffer's 2 GiB, which no slice brings near an L2 (65536 x 2.2 M, 24 per row, N = 256
 // 327 us with four, 361 with eight).
-int auto_slices(int K, int N, double avg_row, bool wide) {
+// On even rows and merge-path parts, whose one or two groups csr_rowblock_wide takes,
+// slices whose columns fill those groups' lanes (128 and more) stay until a share is
+// 3.75 MiB, others until 2.25 (merge-path parts of 192 columns 3.25): 5000^2, 300 per
+// row, N = 256 58 us with four slices, 54 with two; 6000^2, 20 per row, N = 512 15.4 with
+// eight, 13.9 with four; parts of 4200^2, 41 per row, N = 256 17.4 and 15.1; at 4 MiB
+// four win (8192^2, 82 per row 31.7 with two, 30.4).  Uneven rows gain more by the finer
+// ones (power-law 5000^2, N = 256 37.7 with two, 30.3).
+// Slices of 32 columns and more that are no whole lines pay where they bring a share of
+// 4.75 MiB and more to 5 (20000^2, 60 per row, N = 160 68.5 us with two, 61.4 with four;
+// 14000^2, 4.3 MiB, 53.7 and 58.8), but not against whole rows (N = 96 of 24576^2 75 and 80).
+int auto_slices(int K, int N, double avg_row, bool even, bool split, bool wide) {
     const long long b_bytes = static_cast<long long>(K) * N * 4;
     if (b_bytes <= (4LL << 20)) return 1;
     const auto narrowest = [&](int slices) { return !wide && N % (32 * slices) == 0 ? 32 : 64; };
+    const auto over = [&](int slices, int quarter_mib) {  // an XCD's share of B
+        return b_bytes > (static_cast<long long>(quarter_mib) << 18) * slices;
+    };
+    const auto half = [&](int slices) {
+        if (!even && !split) return 8;
+        if (N % (128 * slices) == 0) return 15;
+        return split && N % (64 * slices) == 0 ? 13 : 9;
+    };
     int s = 1;
-    while (s < 8 && ((b_bytes > (4LL << 20) * s && N / (2 * s) >= narrowest(2 * s)) ||
-                     (!wide && b_bytes > (2LL << 20) * s && N / (2 * s) >= 64 && avg_row >= 16.0))) {
+    while (s < 8 && ((over(s, 16) && N / (2 * s) >= narrowest(2 * s)) ||
+                     (!wide && over(s, half(s)) && N / (2 * s) >= 64 && avg_row >= 16.0))) {
         s *= 2;
     }
+    if (!wide && s > 1 && s < 8 && N / (2 * s) >= 32 && over(s, 19) && !over(2 * s, 20)) s *= 2;
     return s;
 }
 
 // Waves of the engine resident at once on the chip: 16 per CU (four 4-wave
 // workgroups) on 256 CUs.
 constexpr long kRoundWaves = 4096;
-
-// Rows whose lengths stay within twice the average (plus a constant for
-// short rows): uniform random rows qualify, power-law rows do not.
-bool rows_even(int M, long long nnz, int max_row) {
-    return max_row > 0 && M > 0 &&
-           max_row <= 2.0 * static_cast<double>(nnz) / M + 32.0;
-}
 
 // Rows per workgroup of the 4-wave row-block launch for even rows: the grid
 // is a whole number of rounds of kRoundWaves waves, one round per ~2 M entry
@@ -1797,7 +1816,8 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
     if (slices == 0) {
         slices = role == CsrRole::Tiled
                      ? 1
-                     : auto_slices(A.num_cols, N, avg, want_groups != 0 || !sbuf);
+                     : auto_slices(A.num_cols, N, avg, rows_even(M, A.nnz, o.max_row_hint),
+                                   split != nullptr, want_groups != 0 || !sbuf);
     }
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     int slice_cols = ceil_div(N, slices);
