@@ -265,24 +265,34 @@ __global__ __launch_bounds__(256) void csr_rows_in_order(
         VT acc = vzero<VEC>();
         // Entries [p, p + cnt) of the chain, cnt <= L, U at a time; entry j is
         // handed out by take(j).
+        auto step = [&](int j0, int cnt, auto take, auto width) {
+            constexpr int W = decltype(width)::value;
+            VT    b[W];
+            float v[W];
+#pragma unroll
+            for (int u = 0; u < W; ++u) {
+                int k;
+                take(min(j0 + u, cnt - 1), k, v[u]);
+                b[u] = *reinterpret_cast<const MT*>(bcol + static_cast<size_t>(k) * N);
+            }
+            if (j0 + W <= cnt) {
+#pragma unroll
+                for (int u = 0; u < W; ++u) acc = fma_vec<VEC>(v[u], b[u], acc);
+            } else {
+#pragma unroll
+                for (int u = 0; u < W; ++u) {
+                    if (j0 + u < cnt) acc = fma_vec<VEC>(v[u], b[u], acc);
+                }
+            }
+        };
+        // Up to four entries left: four loads instead of U (3034 rows of 2.4, N = 320
+        // 6.0 -> 4.8 us).
         auto chain = [&](int cnt, auto take) {
             for (int j0 = 0; j0 < cnt; j0 += U) {
-                VT    b[U];
-                float v[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    int k;
-                    take(min(j0 + u, cnt - 1), k, v[u]);
-                    b[u] = *reinterpret_cast<const MT*>(bcol + static_cast<size_t>(k) * N);
-                }
-                if (j0 + U <= cnt) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) acc = fma_vec<VEC>(v[u], b[u], acc);
+                if (HAND == Hand::Readlane && cnt - j0 <= 4) {  // the wave's one row: uniform
+                    step(j0, cnt, take, std::integral_constant<int, 4>());
                 } else {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        if (j0 + u < cnt) acc = fma_vec<VEC>(v[u], b[u], acc);
-                    }
+                    step(j0, cnt, take, std::integral_constant<int, U>());
                 }
             }
         };
