@@ -1970,10 +1970,12 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     // A B past the L2s whose rows are whole lines: the engine's slices of 32
     // columns beat the row groups on longer rows (65536^2, 40 per row, N = 64 61
     // against 72 us, N = 128 120 against 155 us; 32768^2, 40 per row, N = 256 94
-    // against 131 us) and at any length once B is far larger.  Other widths
+    // against 131 us) and from rows of 8 on once B is far larger (47000 x 110000, 2 per
+    // row, N = 128 13 us in row groups, 14.7).  Other widths
     // cannot be cut that narrow, and there the row groups win on even rows
     // (24576^2, 100 per row, N = 100 65 against 99 us; over 90 inputs with N = 33
-    // .. 250 they lose at most 3%, and at N = 250 on rows of 24 and fewer 15%).
+    // .. 250 they lose at most 3%, and at N = 250 on rows of 24 and fewer 15%), but
+    // not on few (2320 x 6134, 101 per row, N = 180 22.3 us, 12.8 in the engine).
     const double b_mib = static_cast<double>(K) * N / (1 << 18);
     const bool lines = N % (N <= 128 ? 64 : 32) == 0;  // N = 96 has no halves of whole lines
     // Narrow B and rows just too short for more_entry_lanes, on many rows with a B
@@ -1988,14 +1990,16 @@ bool row_groups_pay(int M, int N, int K, double avg_row, int max_row) {
     }
     if (lines && N > 32 && N <= 64 && b_mib >= 16.0 && avg_row >= 16.0) return false;
     if (lines && N > 64 && b_mib > 4.0 &&
-        (avg_row >= (N > 128 ? 16.0 : 24.0) || (N <= 128 && b_mib >= 32.0))) {
+        (avg_row >= (N > 128 ? 16.0 : 24.0) || (N <= 128 && b_mib >= 32.0 && avg_row >= 8.0))) {
         return false;
     }
-    if (N <= 64) return M >= 2048 || avg_row <= 100.0;
+    // Few long rows: at N <= 32 the row groups take 0.55 - 0.8 of the engine's time (1650
+    // inputs of 60 .. 2100 rows of 60 .. 900), at 33 .. 64 0.9 - 1.2.
+    if (N <= 64) return N <= 32 || M >= 2048 || avg_row <= 100.0;
     const bool b_large = avg_row <= 24.0 && b_mib > 4.0 && N >= (N % 32 == 0 ? 64 : 128);
     if (N * avg_row <= 2048.0 || (N <= 256 && b_large)) return true;
     if (max_row > 2.0 * avg_row + 32.0) return false;  // uneven rows
-    if (!lines && N <= 256 && b_mib > 4.0) return true;
+    if (!lines && N <= 256 && b_mib > 4.0 && M >= 4096) return true;
     if (N * avg_row <= 4096.0) return true;
     if (N > 128) return false;
     if (M > 4096 && M <= 8192 && avg_row >= 64.0) return false;

@@ -291,6 +291,15 @@ def test_csr_auto_form(S):
         "rowgroups", "rowgroups", "engine"]
     assert [S.csr_auto_form(_even_rows(S, 65536, 65536, 40), n)[0] for n in (64, 96, 128)] == [
         "engine", "rowgroups", "engine"]
+    # B of 32 MiB and more at N = 128: short rows stay with the row groups; widths
+    # that are no whole lines: few rows take the engine
+    assert [S.csr_auto_form(_even_rows(S, 70000, 70000, p), 128)[0] for p in (3, 7, 8)] == [
+        "rowgroups", "rowgroups", "engine"]
+    assert [S.csr_auto_form(_even_rows(S, m, 6000, 100), 190)[0] for m in (2300, 4095, 4096)] == [
+        "engine", "engine", "rowgroups"]
+    # few long rows: row groups up to N = 32, the engine up to 64
+    assert [S.csr_auto_form(_even_rows(S, 800, 800, 140), n)[0] for n in (1, 16, 32, 33, 64)] == [
+        "rowgroups"] * 3 + ["engine"] * 2
     # narrow B: rows of 20 and more take more entry lanes, shorter ones leave many
     # rows with a B past the L2s to the engine
     forms = lambda m, ns: [S.csr_auto_form(m, n)[0] for n in ns]
