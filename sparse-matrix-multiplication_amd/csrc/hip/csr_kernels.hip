@@ -1488,12 +1488,15 @@ int round_rows_per_block(int M, long long nnz, int slices, int waves) {
 // Rows per workgroup of csr_rowblock on even rows, near rpb: the grid is a whole
 // number of rounds where it would be four or fewer.  512 workgroups of 8 waves fill the
 // chip, and M / 512 rows, rounded down, make a few more of them: 4200 rows of 41, N =
-// 160 12.9 -> 10.0 us, 5000 of 100 21.3 -> 16.8, 3000 of 200, N = 320 44.4 -> 34.9.  Uneven
-// rows keep the finer cut: power-law rows lose as often as they gain (2100 of 60, N =
-// 256 14.5 -> 16.6, 1050 of 100 13.8 -> 12.0).
-int near_round_rows(int M, int rpb, int slices, int waves) {
+// 160 12.9 -> 10.0 us, 5000 of 100 21.3 -> 16.8, 3000 of 200, N = 320 44.4 -> 34.9.  Rows that may
+// be uneven only leave a second round that is not full, and only where a wave has
+// under 32 entries (1000 uniform inputs of 64 K entries and fewer 0.86 -> 0.73 of the time
+// of one group without it, as many power-law ones 0.72 -> 0.70); with more, the finer cut
+// spreads the long rows (power-law 3100 of 100 16.0 us, 20.7 without).
+int near_round_rows(int M, int rpb, int slices, int waves, bool even) {
     const double round = static_cast<double>(kRoundWaves) / waves / slices;  // row blocks
     const double rounds = ceil_div(M, rpb) / round;
+    if (!even) return rounds > 1.0 && rounds < 2.0 ? static_cast<int>(std::ceil(M / round)) : rpb;
     if (rounds > 4.0) return rpb;
     return static_cast<int>(std::ceil(M / (std::max(1.0, std::round(rounds)) * round)));
 }
@@ -1880,7 +1883,9 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
         } else if (rpb <= 0) {
             rpb = static_cast<int>(160.0 * waves / std::max(avg, 1.0) + 0.5);
             rpb = std::min(rpb, M / (slices == 1 ? 512 : 256));
-            if (even_rows && rpb > 0) rpb = near_round_rows(M, rpb, slices, waves);
+            if (rpb > 0 && (even_rows || (vec > 1 && per_wave < 32))) {
+                rpb = near_round_rows(M, rpb, slices, waves, even_rows);
+            }
         }
         rpb = std::max(1, std::min(rpb, kRpCap));
         // 160 entries per wave in eight slices are more threads than a launch
