@@ -1321,6 +1321,22 @@ long sliced_grid(long nblocks, int slices) {
     return slices == 1 ? nblocks : (nblocks + per - 1) / per * 8;
 }
 
+// Most lane groups of a wave, whose ranges cut the rows into pieces that the owner of a
+// row adds one by one.  On explicit partitions and merge-path parts a range has 8
+// entries, or a row where rows are shorter (power-law 2048^2, N = 16 11.1 us with eight
+// waves' reductions, 14.2 with 64 groups of 4 entries; parts of 2.5 per row, N = 272 18.7 us
+// with groups of one row, 29.8 with one group).  Even rows of a few in a workgroup
+// besides take no more than eight pieces a row: 823 rows of 147, N = 48 13.6 -> 6.3 us,
+// 955 of 43, N = 64 8.3 -> 5.2.  Uneven rows of an implicit partition take what fits: there
+// the groups share the long ones (over 700 power-law inputs 4% less time than with ranges
+// of 8 entries).  Two are always taken: csr_rowblock_wide cuts nothing between them.
+int most_groups(int M, double avg, long per_wave, int slices, bool even, bool partition) {
+    if (!even && !partition) return kMaxGroups;
+    long most = per_wave / std::clamp(std::lround(avg), 1L, 8L);
+    if (even) most = std::min<long>(most, M / (slices == 1 ? 512 : 128));
+    return static_cast<int>(std::clamp<long>(most, 2, kMaxGroups));
+}
+
 // Lane groups of a wave: with L = lanes of one row (slice) and p column passes
 // a group takes ceil(L / p) lanes; the pass count with the fewest passes per
 // entry slot (p / groups) wins, fewer passes first.  want: groups asked for.
@@ -1328,19 +1344,14 @@ long sliced_grid(long nblocks, int slices) {
 // N = 160 15.2 us in two passes of 51 entries, 12.2 in one; 2100 of 100, N = 320 25.2
 // and 23.4; 4096 of 60, 60 entries, 11.0 and 11.7), 40 on merge-path
 // parts (power-law 2048^2, mean 64, N = 260 24.6 us in two passes, 29.1 in four; 8192^2,
-// mean 40 50 against 36), and those and explicit partitions take no more than have 8: every part may
-// end in rows whose pieces the owner adds one by one (the first at N = 16 11.1 us
-// with eight waves' reductions, 14.2 with 64 groups of 4 entries).
-void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave) {
+// mean 40 50 against 36).  most: see most_groups.
+void set_groups(RowblockArgs& a, int cols, int vec, int want, long per_wave, int most) {
     const int lanes = ceil_div(cols, vec);
     if (want == 1 || want == 2 || want == 4 || (want == 8 && vec == 4)) {
         a.groups      = want;
         a.group_lanes = kWave / want;
     } else {
         const bool split = a.part.split_rows != nullptr;
-        const int most = split || a.bounds != nullptr
-                             ? static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups))
-                             : kMaxGroups;
         int passes = ceil_div(lanes, kWave), best = passes;
         const auto groups_of = [&](int p) { return std::min(most, kWave / ceil_div(lanes, p)); };
         for (int p = passes + 1; p <= 2 * passes; ++p) {
@@ -1864,9 +1875,10 @@ Error launch_csr_impl(CsrRole role, const CSR& A, const float* B, float* C, int 
         part.nblocks    = split->parts;
     }
     args.bounds = split == nullptr ? bounds : nullptr;
-    set_groups(args, slice_cols, vec, want_groups, per_wave);
     const bool even_rows = split == nullptr && bounds == nullptr && o.rows_per_block <= 0 &&
                            rows_even(M, A.nnz, o.max_row_hint);
+    set_groups(args, slice_cols, vec, want_groups, per_wave,
+               most_groups(M, avg, per_wave, slices, even_rows, split != nullptr || bounds != nullptr));
     // The whole-round grid is for few groups: it leaves more of them too few
     // row pieces each (65536^2, 40 per row, N = 256, eight slices of four groups:
     // 305 us with it, 260 without).
@@ -2071,7 +2083,8 @@ Error launch_csr_khalf(const KHalfPlan& p, const float* B, float* C, hipStream_t
     args.M          = p.M;
     args.N          = N;
     args.slice_cols = N;
-    set_groups(args, N, 4, 0, std::min(args.part.nnz / p.parts[0], args.upper.nnz / p.parts[1]) / 4);
+    const long per_wave = std::min(args.part.nnz / p.parts[0], args.upper.nnz / p.parts[1]) / 4;
+    set_groups(args, N, 4, 0, per_wave, static_cast<int>(std::clamp<long>(per_wave / 8, 1, kMaxGroups)));
     const int grid   = 8 * ceil_div(std::max(p.parts[0], p.parts[1]), 4);
     hipError_t e = args.groups <= 2 ? dispatch_wide<true>(4, args, grid, stream)
                    : fold_windows(args)

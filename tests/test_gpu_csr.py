@@ -687,7 +687,8 @@ def test_row_groups_rounding(S, O, torch):
 
 
 @pytest.mark.parametrize("M,per,N", [(1050, 60, 160), (2100, 100, 320), (525, 9, 77), (4200, 41, 256),
-                                     (7000, 12, 200), (9000, 30, 160), (20000, 20, 160), (4000, 30, 512)])
+                                     (7000, 12, 200), (9000, 30, 160), (20000, 20, 160), (4000, 30, 512),
+                                     (823, 147, 48), (955, 43, 64), (2366, 12, 34), (3034, 3, 320)])
 @pytest.mark.parametrize("pattern", ["even", "uneven"])
 def test_engine_grids_and_slices(S, torch, M, per, N, pattern):
     # Row blocks just over a round of the chip, one and two passes per row, and the
