@@ -1674,6 +1674,13 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
         more = long_log > le_log &&
                more_entry_lanes(M, A.num_cols, N, A.nnz, o.max_row_hint, lc_log, le_log);
         if (more) le_log = long_log;
+        // Rows that may be uneven, up to 16 columns: eight lanes while that is under 2048
+        // waves, for the long rows of a nearly empty chip (power-law 2544 of 2.7, N = 6
+        // 5.5 -> 3.3 us; over 1234 power-law inputs 0.84 -> 0.76 of one float a lane, uniform
+        // ones 0.81 -> 0.80; rows known to be even 1.00).
+        int spare = 3;
+        while (spare > 0 && (static_cast<long>(M) << (lc_log + spare)) * slices > kWave * 2048L) --spare;
+        if (lc_log <= 2 && !rows_even(M, A.nnz, o.max_row_hint)) le_log = std::max(le_log, spare);
     }
     le_log = std::max(0, std::min(le_log, 6 - lc_log));
     const bool b_small = static_cast<long long>(A.num_cols) * N * 4 <= (2LL << 20);

@@ -725,6 +725,33 @@ def test_engine_grids_and_slices(S, torch, M, per, N, pattern):
         check_csr(C.cpu().numpy(), C64.cpu().numpy(), absC.cpu().numpy())
 
 
+@pytest.mark.parametrize("M", [40, 1000, 8191, 8193, 16385, 70000])
+@pytest.mark.parametrize("N", [1, 3, 5, 16])
+def test_row_groups_spare_lanes(S, torch, M, N):
+    # Short rows with a few long ones: eight entry lanes a row, four, two and one as
+    # the rows fill the chip, with and without the longest row as a hint.
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    lens = torch.randint(0, 5, (M,), generator=g, device="cuda")
+    lens[::39] = 90
+    rp = torch.zeros(M + 1, dtype=torch.int32, device="cuda")
+    rp[1:] = lens.cumsum(0)
+    nnz = int(rp[-1])
+    col = torch.randint(0, 500, (nnz,), generator=g, device="cuda", dtype=torch.int32)
+    val = torch.rand(nnz, generator=g, device="cuda") * 2 - 1
+    B = torch.rand((500, N), generator=g, device="cuda") * 2 - 1
+    p = val[:, None].double() * B[col.long()].double()
+    rows = torch.repeat_interleave(torch.arange(M, device="cuda"), lens)
+    C64 = torch.zeros((M, N), dtype=torch.float64, device="cuda").index_add_(0, rows, p)
+    absC = torch.zeros_like(C64).index_add_(0, rows, p.abs())
+    dA = S.DeviceCSR(S.HostCSR(M, 500, rp.cpu().numpy(), col.cpu().numpy(), val.cpu().numpy()))
+    for hint in (0, 90):
+        say(f"csr row groups spare lanes M={M} N={N} hint={hint}")
+        C = torch.full((M, N), float("nan"), device="cuda")
+        S.spmm_tiled_v3_opts(dA, B, S.EngineOptsT(row_groups=1, max_row_hint=hint), C)
+        torch.cuda.synchronize()
+        check_csr(C.cpu().numpy(), C64.cpu().numpy(), absC.cpu().numpy())
+
+
 @pytest.mark.parametrize("N", [100, 130, 198, 250, 499, 512])
 def test_row_groups_column_slices(S, O, torch, N):
     # B past an L2 under rows of up to 24: whole, or in two to eight slices whose
