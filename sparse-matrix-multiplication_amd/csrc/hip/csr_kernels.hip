@@ -1099,6 +1099,9 @@ struct RowGroupArgs {
     int          slices;    // XCD-tied column slices: 1, 2, 4 or 8
     int          slice_cols;
     int          nblocks;   // row blocks (workgroups of one column slice)
+    // Rows of up to few_len entries take 1 << few_log entry lanes of the 1 << le_log.
+    int          few_log = 0;
+    int          few_len = 0;
 };
 
 template <int VEC>
@@ -1179,7 +1182,7 @@ __device__ __forceinline__ typename Vec<VEC>::T row_chunks_sum(
     return acc;
 }
 
-template <int VEC, int U, bool COOP, bool LONG_ROWS>
+template <int VEC, int U, bool COOP, bool LONG_ROWS, bool FEW = false>
 __global__ __launch_bounds__(256) void csr_row_groups(RowGroupArgs a) {
     using VT = typename Vec<VEC>::T;
     const int LC   = 1 << a.lc_log;
@@ -1224,7 +1227,11 @@ __global__ __launch_bounds__(256) void csr_row_groups(RowGroupArgs a) {
             acc = row_chunks_sum<VEC, U>(a, rb, start, g_end, lane & ~(L - 1), gl, e, L, LE, n * 4,
                                          L);
         } else {
-            acc = row_segment_sum<VEC, U>(a, rb, start + e, g_end, LE, n * 4);
+            // FEW: lanes by the row; otherwise the stride is the wave's (500000 rows of 20
+            // 1 - 5% less time).
+            const int lanes = !FEW || g_end - start > a.few_len ? LE : 1 << a.few_log;
+            acc = row_segment_sum<VEC, U>(a, rb, !FEW || e < lanes ? start + e : g_end, g_end, lanes,
+                                          n * 4);
         }
         for (int m = LC; m < L; m <<= 1) acc = xor_add<VEC>(acc, m);
         if (live && !is_long && e == 0 && col) {
@@ -1574,6 +1581,13 @@ int row_group_slices(int K, int N, double avg_row) {
 
 template <int VEC, bool COOP, bool LONG_ROWS>
 hipError_t run_row_groups(const RowGroupArgs& args, int unroll, int grid, hipStream_t stream) {
+    if constexpr (!COOP) {
+        if (args.few_len > 0) {
+            hipLaunchKernelGGL((csr_row_groups<VEC, 2, false, LONG_ROWS, true>), dim3(grid),
+                               dim3(256), 0, stream, args);
+            return hipGetLastError();
+        }
+    }
     if (unroll == 4) {
         hipLaunchKernelGGL((csr_row_groups<VEC, 4, COOP, LONG_ROWS>), dim3(grid), dim3(256), 0,
                            stream, args);
@@ -1653,7 +1667,7 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
     if (slices != 1 && slices != 2 && slices != 4 && slices != 8) slices = 1;
     const int slice_cols = ceil_div(ceil_div(N, slices), vec) * vec;
     const int lc_log = row_group_lc_log(M, slice_cols, vec);
-    int le_log;
+    int le_log, few_log = 0, few_len = 0;
     bool more = false;
     if (o.entry_lanes != 0) {
         if (o.entry_lanes < 0 || o.entry_lanes > 64 || (o.entry_lanes & (o.entry_lanes - 1)) != 0) {
@@ -1677,10 +1691,16 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
         // Rows that may be uneven, up to 16 columns: eight lanes while that is under 2048
         // waves, for the long rows of a nearly empty chip (power-law 2544 of 2.7, N = 6
         // 5.5 -> 3.3 us; over 1234 power-law inputs 0.84 -> 0.76 of one float a lane, uniform
-        // ones 0.81 -> 0.80; rows known to be even 1.00).
+        // ones 0.81 -> 0.80; rows known to be even 1.00).  Rows of two entries a lane and
+        // fewer keep the lanes they had: each lane rounds its first product, so with
+        // eight a row of 3 to 10 would be 4 - 10% further from 64 bits.
         int spare = 3;
         while (spare > 0 && (static_cast<long>(M) << (lc_log + spare)) * slices > kWave * 2048L) --spare;
-        if (lc_log <= 2 && !rows_even(M, A.nnz, o.max_row_hint)) le_log = std::max(le_log, spare);
+        if (lc_log <= 2 && avg < 32.0 && o.unroll == 0 && o.row_groups != 3 && spare > le_log && !rows_even(M, A.nnz, o.max_row_hint)) {
+            few_log = le_log;
+            few_len = 2 << spare;
+            le_log  = spare;
+        }
     }
     le_log = std::max(0, std::min(le_log, 6 - lc_log));
     const bool b_small = static_cast<long long>(A.num_cols) * N * 4 <= (2LL << 20);
@@ -1704,7 +1724,8 @@ Error launch_row_groups(const CSR& A, const float* B, float* C, int N, hipStream
                                   static_cast<int>(std::ceil(std::min(4.0 * avg, 1.0e9))));
     RowGroupArgs args{A.row_ptr, A.col_idx,  A.values,   B,          C,
                       M,         N,          A.num_cols, lc_log,     le_log,
-                      long_len,  slices,     slice_cols, nblocks};
+                      long_len,  slices,     slice_cols, nblocks,    few_log,
+                      few_len};
     // Without a longest-row hint any row may be long: the workgroup-wide pass
     // (one barrier even when no row needs it) is compiled in.
     const bool long_rows = o.max_row_hint <= 0 || o.max_row_hint > long_len;
